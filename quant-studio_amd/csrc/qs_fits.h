@@ -457,46 +457,57 @@ QS_DEV float q3_fit(const float (&x)[N], int nmax, float (&L)[N]) {
 
 // ---- IQ4_XS (iq4_xs.py:23-76) ----
 
-// Bracket table of _best_index (iq4_xs.py:35-39): the LUT values are integers,
-// so #{V <= al} = #{V <= floor(al)}; entry k + 128 (k = -128..127) holds the
-// bracket (V[mu-1], V[mu]) with mu = clamp(#{V <= k}, 1, 15), and mu itself in
-// `mus`. Built by the workgroup in LDS.
-QS_DEV void iq4_build_table(float2* tab, uint8_t* mus) {
-    constexpr float V[16] = {-127.f, -104.f, -83.f, -65.f, -49.f, -35.f, -22.f, -10.f,
-                             1.f,    13.f,   25.f,  38.f,  53.f,  69.f,  89.f,  113.f};
-    for (int e = threadIdx.x; e < 256; e += blockDim.x) {
-        const float k = (float)(e - 128);
-        int mu = 0;
-#pragma unroll
-        for (int i = 0; i < 16; i++) mu += (V[i] <= k) ? 1 : 0;
-        mu = mu < 1 ? 1 : (mu > 15 ? 15 : mu);
-        float lo = V[0], hi = V[1];
-#pragma unroll
-        for (int i = 2; i < 16; i++) {
-            lo = (mu == i) ? V[i - 1] : lo;
-            hi = (mu == i) ? V[i] : hi;
-        }
-        tab[e] = make_float2(lo, hi);
-        mus[e] = (uint8_t)mu;
+// _best_index (iq4_xs.py:35-39) as a table over floor(2 al): the bracket's
+// compare `al - lo < hi - al` is `al < (lo + hi) / 2` (near a midpoint both
+// differences are exact), and the midpoints of the integer LUT are multiples
+// of one half, so the projection only changes where 2 al is an integer. Entry
+// e stands for floor(2 al) = e (e < 512) or e - 1024 (the negative half): a
+// masked floor is always inside the table. `val` holds the LUT value, `idx`
+// its index, one byte each: a search's lookups then fall into the ~60 words
+// around zero, about one per LDS bank.
+// Measured (IQ4_XS with imatrix, bf16 9728x2560): the bracket pair read as
+// float2 at clamp(floor(al)) + 128 and compared took 14 VALU instructions per
+// value and trial and two LDS words, this takes 9 and a byte.
+struct Iq4Tab {
+    alignas(16) int8_t val[1024];
+    alignas(16) uint8_t idx[1024];
+};
+
+constexpr Iq4Tab iq4_make_tab() {
+    constexpr int V[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
+    Iq4Tab t{};
+    for (int e = 0; e < 1024; e++) {
+        const int k = e < 512 ? e : e - 1024;
+        int i = 0;
+        while (i < 15 && V[i] + V[i + 1] <= k) i++;
+        t.val[e] = (int8_t)V[i];
+        t.idx[e] = (uint8_t)i;
     }
+    return t;
 }
 
-// LUT value of _best_index(al): the bracket from the table, then the C
-// midpoint compare `al - lo < hi - al` (strict; NaN takes hi, as the scan)
-QS_DEV float iq4_project(float al, const float2* tab) {
-    const float f = clampf(floorf(al), -128.0f, 127.0f);
-    const float2 e = tab[(int)f + 128];
-    const float d1 = al - e.x, d2 = e.y - al;
-    return d1 < d2 ? e.x : e.y;
+static __device__ const Iq4Tab iq4_tab_const = iq4_make_tab();
+
+// a one-wave workgroup's copy of the table in LDS (16 bytes per lane and half)
+QS_DEV void iq4_load_tab(Iq4Tab& t) {
+    const int lane = (int)threadIdx.x;
+    reinterpret_cast<u32x4*>(t.val)[lane] = reinterpret_cast<const u32x4*>(iq4_tab_const.val)[lane];
+    reinterpret_cast<u32x4*>(t.idx)[lane] = reinterpret_cast<const u32x4*>(iq4_tab_const.idx)[lane];
 }
 
-// LUT index of _best_index(al), from the same table
-QS_DEV int iq4_project_index(float al, const float2* tab, const uint8_t* mus) {
-    const int k = (int)clampf(floorf(al), -128.0f, 127.0f) + 128;
-    const float2 e = tab[k];
-    const int mu = mus[k];
-    const float d1 = al - e.x, d2 = e.y - al;
-    return d1 < d2 ? mu - 1 : mu;
+// floor(v) as an integer, saturating, 0 for NaN (v_cvt_flr_i32_f32)
+QS_DEV int floor_int(float v) { return (int)floorf(v); }
+
+// LUT value of _best_index(al) from al2 = 2 al, for |al| < 256 (a trial's
+// |al| is at most 134). NaN takes entry 0: the sums it enters are NaN or
+// infinite whatever the value.
+QS_DEV float iq4_project(float al2, const Iq4Tab& t) { return (float)t.val[floor_int(al2) & 1023]; }
+
+// LUT index of _best_index(al) for any al; NaN takes index 1, as the bracket
+// compare does
+QS_DEV int iq4_project_index(float al, const Iq4Tab& t) {
+    const float v = al == al ? clampf(2.0f * al, -512.0f, 511.0f) : -200.0f;    // -200: index 1
+    return t.idx[floor_int(v) & 1023];
 }
 
 // _search_scales_eager iq4_xs.py:52-76 for one block of 32. The two sums of
@@ -506,7 +517,7 @@ QS_DEV int iq4_project_index(float al, const float2* tab, const uint8_t* mus) {
 // per SIMD (6-7% faster); the kernels without imatrix were 4% slower at 4
 // waves and stage all 32 (CH = 32, 3 waves).
 template <int CH>
-QS_DEV float iq4_scale_search(const float (&x)[32], const float (&w)[32], const float2* tab) {
+QS_DEV float iq4_scale_search(const float (&x)[32], const float (&w)[32], const Iq4Tab& tab) {
     float amax;
     const float mx = absmax_first(x, amax);
     const bool live = fabsf(mx) >= GROUP_MAX_EPS;
@@ -514,12 +525,13 @@ QS_DEV float iq4_scale_search(const float (&x)[32], const float (&w)[32], const 
     const float d0 = -mxs / -127.0f;
     const float id0 = 1.0f / d0;
     auto sums = [&](float iv, float& sqx, float& sq2) {
+        const float iv2 = 2.0f * iv;      // 2 fl(iv x) = fl(2 iv x)
 #pragma unroll
         for (int c = 0; c < 32; c += CH) {
             float t[CH], u[CH];
 #pragma unroll
             for (int i = 0; i < CH; i++) {
-                const float q = iq4_project(iv * x[c + i], tab);
+                const float q = iq4_project(iv2 * x[c + i], tab);
                 const float wq = w[c + i] * q;
                 t[i] = wq * x[c + i];
                 u[i] = wq * q;

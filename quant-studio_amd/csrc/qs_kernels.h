@@ -768,9 +768,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     // LDS is what limits this kernel's residency: the imatrix path stages x^2
     // for sigma2 half the wave's superblocks at a time, the other stages none
     __shared__ SbLds<SPW, BYTES, IMAT ? SPW / 2 : 1> s;
-    __shared__ float2 iq4tab[256];
-    __shared__ uint8_t iq4mu[256];
-    iq4_build_table(iq4tab, iq4mu);
+    __shared__ Iq4Tab iq4tab;
+    iq4_load_tab(iq4tab);
     const SbPos p = sb_pos<LPS, 32>(a.n_units, a.units_per_row, a.stride);
     const int slot = p.slot, g = p.g;
     float x[32], w[32];
@@ -797,7 +796,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const float dl = d * lsf;
     const float idl = dl != 0.0f ? 1.0f / dl : 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; i++) s.L[slot][32 * g + i] = (uint8_t)iq4_project_index(idl * x[i], iq4tab, iq4mu);
+    for (int i = 0; i < 32; i++) s.L[slot][32 * g + i] = (uint8_t)iq4_project_index(idl * x[i], iq4tab);
     s.ls[slot][g] = (int)(lsf + 32.0f);
     if (g == 0) s.hdr[slot][0] = __builtin_bit_cast(float, f16_bits(d));
     wave_sync();
@@ -840,9 +839,8 @@ template <int SRC, bool IMAT, int SQ>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_iq4_nl(KArgs a) {
     constexpr int BYTES = 18;
     __shared__ __attribute__((aligned(16))) uint8_t stage[64 * BYTES];
-    __shared__ float2 iq4tab[256];
-    __shared__ uint8_t iq4mu[256];
-    iq4_build_table(iq4tab, iq4mu);
+    __shared__ Iq4Tab iq4tab;
+    iq4_load_tab(iq4tab);
     const int lane = threadIdx.x;
     const int64_t b0 = (int64_t)blockIdx.x * 64;
     int64_t b = b0 + lane;
@@ -867,8 +865,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     o[1] = (uint8_t)(h >> 8);
 #pragma unroll
     for (int j = 0; j < 16; j++) {
-        const int lo = iq4_project_index(id * x[j], iq4tab, iq4mu);
-        const int hi = iq4_project_index(id * x[j + 16], iq4tab, iq4mu);
+        const int lo = iq4_project_index(id * x[j], iq4tab);
+        const int hi = iq4_project_index(id * x[j + 16], iq4tab);
         o[2 + j] = (uint8_t)(lo | (hi << 4));
     }
     wave_sync();
