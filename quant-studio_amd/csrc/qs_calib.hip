@@ -5,8 +5,12 @@
 // instructions per CU per clock; an SGPR operand in every instruction halves
 // that, so the operands here are per-lane values. k_copy_stream: a streaming
 // copy, the HBM rate the 32-value formats are compared with. Built into their
-// own library (libqs_calib.so) and used only by bench.py.
+// own library (libqs_calib.so) and used only by bench.py and the tests.
+// k_recip: the two properties the quantizers' division rests on, over every
+// mantissa.
 #include <hip/hip_runtime.h>
+
+#include "qs_device.h"
 
 namespace {
 
@@ -54,9 +58,47 @@ __global__ __launch_bounds__(256) void k_copy_stream(const u32x4* __restrict__ s
     }
 }
 
+// One thread per mantissa of b = m 2^e: the largest |1 - b recip(b)| m 2^23 (in
+// f64, where the product of two 24-bit mantissas is exact) over every mantissa
+// but the last 64, as the bits of a non-negative float, and the number of wrong
+// quotients: every dividend mantissa by the last 64 divisors, and a small set of
+// dividends by every divisor.
+__global__ __launch_bounds__(256) void k_recip(int e, uint32_t* worst, uint32_t* differ) {
+    const uint32_t mant = blockIdx.x * 256u + threadIdx.x;          // 2^23 threads
+    const float m = __uint_as_float(0x3f800000u | mant);
+    const float b = ldexpf(m, e);
+    const float y = qs::recip(b);
+    const double err = fabs(1.0 - (double)b * (double)y) * (double)m * 8388608.0;
+    if (mant < 0x7fffc0u) atomicMax(worst, __float_as_uint((float)err));
+    uint32_t bad = 0;
+    for (uint32_t i = 0; i < 64; i++) {
+        const float last = ldexpf(__uint_as_float(0x3fffffc0u + i), e);
+        bad += __float_as_uint(qs::quotient(m, last, qs::recip(last))) != __float_as_uint(m / last);
+    }
+    uint32_t h = mant * 2654435761u + 12345u;
+    for (int i = 0; i < 16; i++) {
+        h = h * 1664525u + 1013904223u;
+        // mantissas at both ends of the range and spread over it
+        const uint32_t am = i == 0 ? 0u : i == 1 ? 0x7fffffu : i == 2 ? mant : i == 3 ? mant + 1u : h >> 9;
+        const float a = ldexpf(__uint_as_float(0x3f800000u | (am & 0x7fffffu)), (int)(h >> 4) % 30 - 15);
+        bad += __float_as_uint(qs::quotient(a, b, y)) != __float_as_uint(a / b);
+    }
+    if (bad) atomicAdd(differ, bad);
+}
+
 }  // namespace
 
 extern "C" {
+
+// Check qs::recip and qs::quotient over every mantissa of a divisor of exponent
+// e (-60 .. 60) on hip_stream; result: two device words, zeroed by the caller
+// (the worst |1 - b recip(b)| m 2^23 as float bits, the differing quotients).
+int qs_calib_recip(int e, unsigned* result, void* hip_stream) {
+    if (!result || e < -60 || e > 60) return -22;
+    hipLaunchKernelGGL(k_recip, dim3((1u << 23) / 256), dim3(256), 0, static_cast<hipStream_t>(hip_stream), e,
+                       result, result + 1);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+}
 
 // Copy nbytes (a multiple of 16; both pointers 16-byte aligned) on hip_stream.
 int qs_calib_copy(const void* src, void* dst, long long nbytes, void* hip_stream) {

@@ -27,8 +27,20 @@ struct QkxResult {
 };
 
 // make_qkx_quants_eager kq_common.py:51-96 for one group of N values.
-// SPEC: divide the next candidate's inverse scale during the error pass (below).
-template <int N, bool MAD, bool SPEC = false>
+//
+// The loop is bound by VALU issue: 16 instructions per value and candidate,
+// two of them (the rounding and the clamp) at half rate, and the divisions.
+// Those are a reciprocal of D shared by the scale and the min, a reciprocal
+// of the accepted candidate's range mx - mn kept for the candidates that
+// follow, and one quotient per candidate for its inverse scale; when a lane's
+// operands leave the range in which quotient() is the IEEE division, the wave
+// repeats the candidate's divisions with `/` (same bits where both are valid,
+// so the choice is the wave's). issue_break() keeps the paired issue alive.
+// Measured on random groups, clocks per candidate and wave on one SIMD: N = 32
+// 1,797 with five `/` -> 1,395 with shared reciprocals -> 1,269 with the issue
+// breaks (525 instructions at the paired rate would take 1,120); N = 16 871 ->
+// 789 -> 689.
+template <int N, bool MAD>
 QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& steps, float fmax) {
     float mn = x[0], mx = x[0];
 #pragma unroll
@@ -56,34 +68,29 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
         d = d - x[i];
         t[i] = w[i] * (MAD ? fabsf(d) : d * d);
     }
-    float best = tree_sum(t);
+    // a group with mx == mn accepts nothing (its D is 0 or NaN, and no error is
+    // below -inf)
+    float best = degen ? -__builtin_inff() : tree_sum(t);
 
+    // A range mx - mn, a scale or a min within [LO, HI] and D within [DLO, DHI]
+    // keep every division in quotient()'s range: the numerators of scale and min
+    // are then at least 2^-96, the inverse scales (the candidates' numerators
+    // are 0.5 .. 33) within 2^+-61.
+    constexpr float LO = 0x1p-36f, HI = 0x1p60f, DLO = 0x1p-60f, DHI = 0x1p36f;
+    float y = recip(den);                     // of the current range
+    // lanes whose current range needs `/` (a mask, so it stays in scalar registers)
+    uint64_t far = wave_mask(!(den >= LO && den <= HI));
     // 16-value groups load each step one candidate ahead, so the scalar
     // load's latency is not waited for at the top of every candidate (Q2_K
-    // 2-6% faster). With SPEC the next candidate's inverse scale is divided
-    // both ways while this candidate's error pass runs, for a kept min
-    // (mx - mn) and for this candidate's min should it be accepted
-    // (mx - this_min), so no division heads the next candidate; the quotients
-    // are the ones dividing after the accept gives. Q4_K / Q5_K with imatrix
-    // (37 candidates) run 1.4-1.9% faster that way; without imatrix they ran
-    // 1.4-2.3% slower and 16-value groups 5-9% slower (one more division per
-    // candidate weighs more there), so only the former use it.
-    static_assert(!SPEC || N == 32, "SPEC is timed for 32-value groups only");
+    // 2-6% faster)
     constexpr bool AHEAD = N == 16;
     float step_next = steps.v[0];
-    float isc_keep = SPEC ? step_next / den : 0.0f, isc_acc = isc_keep;
-    bool accepted = false;
 #pragma unroll 1
     for (int s = 0; s < steps.n; s++) {
-        float isc;
-        if constexpr (SPEC) {
-            isc = accepted ? isc_acc : isc_keep;
-        } else {
-            const float step = AHEAD ? step_next : steps.v[s];
-            if constexpr (AHEAD) step_next = steps.v[s + 1 < 40 ? s + 1 : 39];
-            den = degen ? 1.0f : mx - mn;
-            isc = step / den;
-        }
+        const float step = AHEAD ? step_next : steps.v[s];
+        if constexpr (AHEAD) step_next = steps.v[s + 1 < 40 ? s + 1 : 39];
+        float isc = quotient(step, den, y);
+        if (far != 0) isc = step / den;
         // the three tree sums are formed 8 values at a time (the tree over N
         // is the trees over its 8-value blocks, then the tree over the block
         // sums), so only one block of products is live at once
@@ -100,25 +107,38 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
                 b[j] = a[j] * La[i];
                 c[j] = a[j] * x[i];
             }
+            issue_break(a[3]);
             sa[k] = tree_sum(a);
             sb[k] = tree_sum(b);
             sc[k] = tree_sum(c);
+            issue_break(sc[k]);
         }
         const float sum_l = tree_sum(sa), sum_l2 = tree_sum(sb), sum_xl = tree_sum(sc);
         const float D = sum_w * sum_l2 - sum_l * sum_l;
         const float Dsafe = D > 0 ? D : 1.0f;
-        float this_scale = (sum_w * sum_xl - sum_x * sum_l) / Dsafe;
-        float this_min = (sum_l2 * sum_x - sum_l * sum_xl) / Dsafe;
+        const float num_s = sum_w * sum_xl - sum_x * sum_l, num_m = sum_l2 * sum_x - sum_l * sum_xl;
+        const float yd = recip(Dsafe);
+        float this_scale = quotient(num_s, Dsafe, yd), this_min = quotient(num_m, Dsafe, yd);
+        const float q_s = fabsf(this_scale), q_m = fabsf(this_min);
         if (this_min > 0) {
             this_scale = sum_xl / fmaxf(sum_l2, F32_TINY);
             this_min = 0.0f;
         }
-        float next_keep = 0.0f, next_acc = 0.0f;
-        if constexpr (SPEC) {
-            const float step = steps.v[s + 1 < 40 ? s + 1 : 39];
-            next_keep = step / (degen ? 1.0f : mx - mn);
-            next_acc = step / (degen ? 1.0f : mx - this_min);
+        float den_acc = mx - this_min;
+        // only a candidate that can be accepted has to be exact
+        const bool live = D > 0;
+        const float q_lo = fminf(fminf(q_s, q_m), den_acc), q_hi = fmaxf(fmaxf(q_s, q_m), den_acc);
+        const bool out = live && !(q_lo >= LO && q_hi <= HI && D >= DLO && D <= DHI);
+        if (wave_any(out)) {
+            this_scale = num_s / Dsafe;
+            this_min = num_m / Dsafe;
+            if (this_min > 0) {
+                this_scale = sum_xl / fmaxf(sum_l2, F32_TINY);
+                this_min = 0.0f;
+            }
+            den_acc = mx - this_min;
         }
+        const float y_acc = recip(den_acc);
         float se[NB];
 #pragma unroll
         for (int k = 0; k < NB; k++) {
@@ -131,18 +151,22 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
                 d = d - x[i];
                 e8[j] = w[i] * (MAD ? fabsf(d) : d * d);
             }
+            issue_break(e8[3]);
             se[k] = tree_sum(e8);
+            issue_break(se[k]);
         }
         const float cur = tree_sum(se);
-        accepted = D > 0 && cur < best && !degen;
-        isc_keep = next_keep;
-        isc_acc = next_acc;
-        if (accepted) {
+        const bool accept = live && cur < best;
+        const uint64_t acc = wave_mask(accept);
+        far = (far & ~acc) | (wave_mask(out) & acc);
+        if (accept) {
             best_isc = isc;
             best_mn = mn;
             scale = this_scale;
             mn = this_min;
             best = cur;
+            den = den_acc;
+            y = y_acc;
         }
     }
     QkxResult r;

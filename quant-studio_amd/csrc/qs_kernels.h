@@ -341,12 +341,11 @@ QS_DEV float sb_sumsq_halves(float (*v)[QK_K], float (*tmp)[40], const float (&x
 // ------------------------------------------------------------------
 template <int SRC, bool IMAT, int NMAX, int SQ>
 // SQ: the host whose square-root rounding the weights take (SQ_*).
-// Occupancy: the imatrix variant (143 VGPRs) runs 3 waves per SIMD; the other
-// (131) is held to 128 for a fourth wave: its 6 spilled registers cost one
-// scratch store on an accepted candidate and reloads after the candidate
-// loop (measured 5% faster). Held to 128, the imatrix variant spills inside
-// the loop and is 7% slower.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(IMAT ? 3 : 4))) void k_q45_k(KArgs a, Steps steps, QpSteps qps) {
+// Occupancy: 3 waves per SIMD for both variants (135-166 VGPRs). The loop
+// issues at the paired rate from 2 waves up, so the variant without imatrix
+// is no longer held to 128 registers for a fourth wave (12 spilled: 82.6 us for
+// Q5_K f16 2560x4096, 67.3 us at 3 waves).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_q45_k(KArgs a, Steps steps, QpSteps qps) {
     constexpr int LPS = 8, SPW = 8, BYTES = NMAX == 15 ? 144 : 176;
     constexpr float FMAX = (float)NMAX;
     // the imatrix path stages x^2 of all 8 superblocks for sigma2; the other
@@ -373,7 +372,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(IMAT ? 3 : 4
         for (int i = 0; i < 32; i++) w[i] = av + fabsf(x[i]);
     }
 
-    const QkxResult r = qkx_fit<32, false, IMAT>(x, w, steps, FMAX);
+    const QkxResult r = qkx_fit<32, false>(x, w, steps, FMAX);
     s.sc[slot][g] = r.scale;
     s.mn[slot][g] = r.the_min;
     if constexpr (IMAT) s.sw[slot][g] = cascade8_sum(w);
