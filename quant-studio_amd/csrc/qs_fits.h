@@ -183,6 +183,48 @@ QS_DEV float qkx_level(const QkxResult& r, float x, float fmax) {
     return r.degen ? 0.0f : clampf(rintf(r.isc * (x - r.mn)), 0.0f, fmax);
 }
 
+// Final levels of a group: clamp(rint(t[i] / d), lo, hi) for the N values of one
+// divisor, from one reciprocal (5 full-rate instructions a value for the
+// division instead of 10 at mostly half rate). The rounded quotient is IEEE's
+// where |t| >= 2^-96; below that, with |d| >= 2^-36, both quotients round to
+// zero. Waves holding a divisor or value outside the range divide with `/`.
+// Lanes with d = 0 get no meaningful levels.
+template <int N>
+QS_DEV void quotient_levels(const float (&t)[N], float d, float lo, float hi, float (&v)[N]) {
+    const float y = recip(d);
+    float m = fabsf(t[0]);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        m = fmaxf(m, fabsf(t[i]));
+        v[i] = clampf(rintf(quotient(t[i], d, y)), lo, hi);
+        if (i % 4 == 3) issue_break(v[i]);
+    }
+    const float ad = fabsf(d);
+    const bool in = m <= 0x1p60f && ad >= 0x1p-36f && ad <= 0x1p36f;
+    if (wave_any(!in && d != 0.0f)) {
+#pragma unroll
+        for (int i = 0; i < N; i++) v[i] = clampf(rintf(t[i] / d), lo, hi);
+    }
+}
+
+// N levels (integers 0 .. 255) as bytes to N consecutive bytes of LDS at a
+// 16-byte boundary: one conversion and merge per value, 16-byte stores (one
+// byte store per value took a quarter of the requantization)
+template <int N>
+QS_DEV void store_levels(const float (&v)[N], uint8_t* o) {
+#pragma unroll
+    for (int q = 0; q < N / 16; q++) {
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            w[j] = 0;
+#pragma unroll
+            for (int b = 0; b < 4; b++) w[j] = __builtin_amdgcn_cvt_pk_u8_f32(v[16 * q + 4 * j + b], b, w[j]);
+        }
+        reinterpret_cast<u32x4*>(o)[q] = u32x4{w[0], w[1], w[2], w[3]};
+    }
+}
+
 // make_qp_quants_eager kq_common.py:99-141, in three parts: qp_trial (one
 // trial's weighted error), qp_finish (levels, sums and refinement passes for
 // the chosen iscale) and the choice between them, made by qp_fit on one lane

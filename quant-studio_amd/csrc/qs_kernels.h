@@ -303,6 +303,13 @@ struct alignas(16) SbLds {
     int ls[SPW][16], lm[SPW][16];
 };
 
+// a word to a 2-byte boundary of LDS
+QS_DEV void store_u16x2(uint8_t* o, uint32_t v) {
+    uint16_t* p = reinterpret_cast<uint16_t*>(o);
+    p[0] = (uint16_t)v;
+    p[1] = (uint16_t)(v >> 16);
+}
+
 // finish: every valid superblock of the wave has its bytes in s.out
 template <int SPW, int BYTES, int VSB>
 QS_DEV void sb_store(const SbLds<SPW, BYTES, VSB>& s, const KArgs& a) {
@@ -428,47 +435,44 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     }
 
     const float dg = d16 * (float)(ls & 63), mg = m16 * (float)(lm & 63);
+    {
+        float t[32], v[32];
 #pragma unroll
-    for (int i = 0; i < 32; i++) {
-        float v;
-        if (dg != 0.0f) {
-            const float t = x[i] + mg;
-            v = clampf(rintf(t / dg), 0.0f, FMAX);
-        } else {
-            v = qkx_level(r, x[i], FMAX);
+        for (int i = 0; i < 32; i++) t[i] = x[i] + mg;
+        quotient_levels(t, dg, 0.0f, FMAX, v);
+        if (wave_any(dg == 0.0f)) {
+#pragma unroll
+            for (int i = 0; i < 32; i++) v[i] = dg == 0.0f ? qkx_level(r, x[i], FMAX) : v[i];
         }
-        s.L[slot][32 * g + i] = (uint8_t)(int)v;
-    }
-    if (g == 0) {
-        s.hdr[slot][2] = __builtin_bit_cast(float, f16_bits(d16));
-        s.hdr[slot][3] = __builtin_bit_cast(float, f16_bits(m16));
+        store_levels(v, s.L[slot] + 32 * g);
     }
     wave_sync();
 
-    // pack (q4_k.py:70-78, q5_k.py:70-81)
-    const uint8_t* L = s.L[slot];
+    // pack (q4_k.py:70-78, q5_k.py:70-81), a word of four levels at a time
+    const uint32_t* L = reinterpret_cast<const uint32_t*>(s.L[slot]);
     const int* LS = s.ls[slot];
     const int* LM = s.lm[slot];
     uint8_t* o = s.out + slot * BYTES;
-    const uint32_t dbits = __builtin_bit_cast(uint32_t, s.hdr[slot][2]);
-    const uint32_t mbits = __builtin_bit_cast(uint32_t, s.hdr[slot][3]);
-    for (int bi = g; bi < BYTES; bi += LPS) {
-        uint32_t v;
-        if (bi < 2) v = dbits >> (8 * bi);
-        else if (bi < 4) v = mbits >> (8 * (bi - 2));
-        else if (bi < 8) { const int j = bi - 4; v = LS[j] | ((LS[4 + j] >> 4) << 6); }
-        else if (bi < 12) { const int j = bi - 8; v = LM[j] | ((LM[4 + j] >> 4) << 6); }
-        else if (bi < 16) { const int j = bi - 12; v = (LS[4 + j] & 15) | ((LM[4 + j] & 15) << 4); }
-        else if (NMAX == 31 && bi < 48) {
-            const int l = bi - 16;
-            v = 0;
+    uint32_t* o4 = reinterpret_cast<uint32_t*>(o);       // BYTES and the staging are multiples of 16
+    if (g == 0) o4[0] = f16_bits(d16) | (f16_bits(m16) << 16);
+    if (g < 4) {
+        o[4 + g] = (uint8_t)(LS[g] | ((LS[4 + g] >> 4) << 6));
+        o[8 + g] = (uint8_t)(LM[g] | ((LM[4 + g] >> 4) << 6));
+        o[12 + g] = (uint8_t)((LS[4 + g] & 15) | ((LM[4 + g] & 15) << 4));
+    }
+    if constexpr (NMAX == 31) {
+        uint32_t h = 0;                                   // qh: bit 4 of the level of sub-block sb at bit sb
 #pragma unroll
-            for (int sb = 0; sb < 8; sb++) v |= ((L[32 * sb + l] >> 4) & 1u) << sb;
-        } else {
-            const int t = bi - (NMAX == 31 ? 48 : 16), j = t >> 5, l = t & 31;
-            v = (L[64 * j + l] & 15u) | ((L[64 * j + 32 + l] & 15u) << 4);
-        }
-        o[bi] = (uint8_t)v;
+        for (int sb = 0; sb < 8; sb++) h |= ((L[8 * sb + g] >> 4) & 0x01010101u) << sb;
+        o4[4 + g] = h;
+    }
+    {
+        // lane g: 16 bytes of qs, the low nibbles of 16 levels of sub-block 2j and of 2j + 1
+        const int j = g >> 1, l = 4 * (g & 1);
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(L + 16 * j + l);
+        const u32x4 hi = *reinterpret_cast<const u32x4*>(L + 16 * j + 8 + l);
+        *reinterpret_cast<u32x4*>(o4 + (NMAX == 31 ? 12 : 4) + 8 * j + l) =
+            (lo & 0x0f0f0f0fu) | ((hi & 0x0f0f0f0fu) << 4);
     }
     wave_sync();
     sb_store(s, a);
@@ -502,38 +506,42 @@ __global__ __launch_bounds__(64) void k_q6_k(KArgs a, Steps steps) {
     int sc8 = (int)fminf(rintf(iscale * r.scale), 127.0f);
     sc8 = ((sc8 & 0xFF) ^ 0x80) - 0x80;
     const float dq = d16 * (float)sc8;
+    {
+        float v[16];
+        quotient_levels(x, dq, -32.0f, 31.0f, v);
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        float v;
-        if (dq != 0.0f) v = clampf(rintf(x[i] / dq), -32.0f, 31.0f) + 32.0f;
-        else v = qx_level(r, x[i], 32.0f);
-        s.L[slot][16 * g + i] = live ? (uint8_t)(int)v : (uint8_t)0;
+        for (int i = 0; i < 16; i++) v[i] = v[i] + 32.0f;
+        if (wave_any(dq == 0.0f)) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = dq == 0.0f ? qx_level(r, x[i], 32.0f) : v[i];
+        }
+        if (wave_any(!live)) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = live ? v[i] : 0.0f;
+        }
+        store_levels(v, s.L[slot] + 16 * g);
     }
-    s.ls[slot][g] = live ? sc8 : 0;
-    if (g == 0) s.hdr[slot][0] = __builtin_bit_cast(float, f16_bits(d16));
     wave_sync();
 
-    // pack (q6_k.py:55-64)
-    const uint8_t* L = s.L[slot];
+    // pack (q6_k.py:55-64), a word of four levels at a time; the block's fields
+    // are 2-byte aligned
+    const uint32_t* L = reinterpret_cast<const uint32_t*>(s.L[slot]);
     uint8_t* o = s.out + slot * BYTES;
-    const uint32_t dbits = __builtin_bit_cast(uint32_t, s.hdr[slot][0]);
-    for (int bi = g; bi < BYTES; bi += LPS) {
-        uint32_t v;
-        if (bi < 128) {
-            const int h = bi >> 6, rr = bi & 63;
-            const uint8_t* q = L + 128 * h + (rr & 31) + (rr >= 32 ? 32 : 0);
-            v = (q[0] & 15u) | ((q[64] & 15u) << 4);
-        } else if (bi < 192) {
-            const int t = bi - 128, h = t >> 5, l = t & 31;
-            const uint8_t* q = L + 128 * h + l;
-            v = (q[0] >> 4) | ((q[32] >> 4) << 2) | ((q[64] >> 4) << 4) | ((q[96] >> 4) << 6);
-        } else if (bi < 208) {
-            v = (uint32_t)s.ls[slot][bi - 192] & 0xFFu;
-        } else {
-            v = dbits >> (8 * (bi - 208));
-        }
-        o[bi] = (uint8_t)v;
+    const int h = g >> 3, l = g & 7;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const uint32_t* q = L + 32 * h + 2 * l + k;       // ql bytes 8 g + 4 k .. + 3
+        store_u16x2(o + 8 * g + 4 * k, (q[0] & 0x0f0f0f0fu) | ((q[16] & 0x0f0f0f0fu) << 4));
     }
+    {
+        const uint32_t* q = L + 32 * h + l;               // qh bytes 4 g .. + 3
+        uint32_t v = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v |= ((q[8 * i] >> 4) & 0x03030303u) << (2 * i);
+        store_u16x2(o + 128 + 4 * g, v);
+    }
+    o[192 + g] = (uint8_t)(live ? sc8 : 0);
+    if (g == 0) *reinterpret_cast<uint16_t*>(o + 208) = (uint16_t)f16_bits(d16);
     wave_sync();
     sb_store(s, a);
 }
@@ -601,45 +609,38 @@ __global__ __launch_bounds__(64) void k_q3_k(KArgs a, Steps steps4, Steps steps3
     }
 
     const float dq = d16 * (float)(ls6 - 32);
+    {
+        float v[16];
+        quotient_levels(x, dq, -4.0f, 3.0f, v);
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const float v = dq != 0.0f ? clampf(rintf(x[i] / dq), -4.0f, 3.0f) + 4.0f : Lg[i];
-        s.L[slot][16 * g + i] = (uint8_t)(int)v;
+        for (int i = 0; i < 16; i++) v[i] = dq != 0.0f ? v[i] + 4.0f : Lg[i];
+        store_levels(v, s.L[slot] + 16 * g);
     }
-    wave_sync();
     s.ls[slot][g] = ls6;
-    if (g == 0) s.hdr[slot][1] = __builtin_bit_cast(float, f16_bits(d16));
     wave_sync();
 
-    // pack (q3_k.py:61-77)
-    const uint8_t* L = s.L[slot];
+    // pack (q3_k.py:61-77), words of levels; the block's fields are 2-byte aligned
+    const uint32_t* L = reinterpret_cast<const uint32_t*>(s.L[slot]);
     const int* LS = s.ls[slot];
     uint8_t* o = s.out + slot * BYTES;
-    const uint32_t dbits = __builtin_bit_cast(uint32_t, s.hdr[slot][1]);
-    for (int bi = g; bi < BYTES; bi += LPS) {
-        uint32_t v = 0;
-        if (bi < 32) {
+    {
+        uint32_t v = 0;                                   // hmask bytes 2 g, 2 g + 1: bit 2 of the levels
 #pragma unroll
-            for (int b = 0; b < 8; b++) v |= (L[32 * b + bi] > 3 ? 1u : 0u) << b;
-        } else if (bi < 96) {
-            const int t = bi - 32, h = t >> 5, l = t & 31;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint32_t q = L[128 * h + 32 * i + l];
-                q = q > 3 ? q - 4 : q;
-                v |= q << (2 * i);
-            }
-        } else if (bi < 104) {
-            const int j = bi - 96;
-            v = (LS[j] & 15) | ((LS[j + 8] & 15) << 4);
-        } else if (bi < 108) {
-            const int i = bi - 104;
-            v = (LS[i] >> 4) | ((LS[4 + i] >> 4) << 2) | ((LS[8 + i] >> 4) << 4) | ((LS[12 + i] >> 4) << 6);
-        } else {
-            v = dbits >> (8 * (bi - 108));
-        }
-        o[bi] = (uint8_t)v;
+        for (int b = 0; b < 8; b++)
+            v |= (((uint32_t)reinterpret_cast<const uint16_t*>(L)[16 * b + g] >> 2) & 0x0101u) << b;
+        *reinterpret_cast<uint16_t*>(o + 2 * g) = (uint16_t)v;
     }
+    {
+        const uint32_t* q = L + 32 * (g >> 3) + (g & 7);  // qs bytes 4 g .. + 3: bits 0-1
+        uint32_t v = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v |= (q[8 * i] & 0x03030303u) << (2 * i);
+        store_u16x2(o + 32 + 4 * g, v);
+    }
+    if (g < 8) o[96 + g] = (uint8_t)((LS[g] & 15) | ((LS[g + 8] & 15) << 4));
+    if (g < 4)
+        o[104 + g] = (uint8_t)((LS[g] >> 4) | ((LS[4 + g] >> 4) << 2) | ((LS[8 + g] >> 4) << 4) | ((LS[12 + g] >> 4) << 6));
+    if (g == 0) *reinterpret_cast<uint16_t*>(o + 108) = (uint16_t)f16_bits(d16);
     wave_sync();
     sb_store(s, a);
 }
@@ -719,41 +720,29 @@ __global__ __launch_bounds__(64) void k_q2_k(KArgs a, Steps steps, QpSteps qps) 
     }
     const int scb = (ls | (lm << 4)) & 0xFF;
     const float dg = d16 * (float)(scb & 15), mg = m16 * (float)(scb >> 4);
+    {
+        float t[16], v[16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        float v;
-        if (dg != 0.0f) {
-            const float t = x[i] + mg;
-            v = clampf(rintf(t / dg), 0.0f, 3.0f);
-        } else {
-            v = qkx_level(r, x[i], 3.0f);
+        for (int i = 0; i < 16; i++) t[i] = x[i] + mg;
+        quotient_levels(t, dg, 0.0f, 3.0f, v);
+        if (wave_any(dg == 0.0f)) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = dg == 0.0f ? qkx_level(r, x[i], 3.0f) : v[i];
         }
-        s.L[slot][16 * g + i] = (uint8_t)(int)v;
-    }
-    wave_sync();
-    s.ls[slot][g] = scb;
-    if (g == 0) {
-        s.hdr[slot][2] = __builtin_bit_cast(float, f16_bits(d16));
-        s.hdr[slot][3] = __builtin_bit_cast(float, f16_bits(m16));
+        store_levels(v, s.L[slot] + 16 * g);
     }
     wave_sync();
 
-    // pack (q2_k.py:74-80)
-    const uint8_t* L = s.L[slot];
+    // pack (q2_k.py:74-80), a word of four levels at a time
     uint8_t* o = s.out + slot * BYTES;
-    const uint32_t dbits = __builtin_bit_cast(uint32_t, s.hdr[slot][2]);
-    const uint32_t mbits = __builtin_bit_cast(uint32_t, s.hdr[slot][3]);
-    for (int bi = g; bi < BYTES; bi += LPS) {
-        uint32_t v = 0;
-        if (bi < 16) v = (uint32_t)s.ls[slot][bi];
-        else if (bi < 80) {
-            const int t = bi - 16, h = t >> 5, l = t & 31;
+    uint32_t* o4 = reinterpret_cast<uint32_t*>(o);        // BYTES is a multiple of 4
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(s.L[slot]) + 32 * (g >> 3) + (g & 7);
+    uint32_t v = 0;                                       // qs bytes 4 g .. + 3
 #pragma unroll
-            for (int i = 0; i < 4; i++) v |= (uint32_t)L[128 * h + 32 * i + l] << (2 * i);
-        } else if (bi < 82) v = dbits >> (8 * (bi - 80));
-        else v = mbits >> (8 * (bi - 82));
-        o[bi] = (uint8_t)v;
-    }
+    for (int i = 0; i < 4; i++) v |= q[8 * i] << (2 * i);
+    o4[4 + g] = v;
+    o[g] = (uint8_t)scb;
+    if (g == 0) o4[20] = f16_bits(d16) | (f16_bits(m16) << 16);
     wave_sync();
     sb_store(s, a);
 }
