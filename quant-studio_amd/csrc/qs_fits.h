@@ -381,7 +381,14 @@ QS_DEV float2 qx_trial(const float (&x)[N], const float (&w)[N], float isc, floa
         t[i] = (w[i] * x[i]) * La;
         u[i] = (w[i] * La) * La;
     }
-    return make_float2(seq_sum(t), seq_sum(u));
+    float st = t[0], su = u[0];
+#pragma unroll
+    for (int i = 1; i < N; i++) {
+        st = st + t[i];
+        su = su + u[i];
+        if (i == N / 2) issue_break(st);
+    }
+    return make_float2(st, su);
 }
 
 template <int N>
@@ -562,7 +569,11 @@ QS_DEV void iq4_load_tab(Iq4Tab& t) {
 }
 
 // floor(v) as an integer, saturating, 0 for NaN (v_cvt_flr_i32_f32)
-QS_DEV int floor_int(float v) { return (int)floorf(v); }
+QS_DEV int floor_int(float v) {
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));     // the compiler takes two instructions
+    return r;
+}
 
 // LUT value of _best_index(al) from al2 = 2 al, for |al| < 256 (a trial's
 // |al| is at most 134). NaN takes entry 0: the sums it enters are NaN or
@@ -574,6 +585,21 @@ QS_DEV float iq4_project(float al2, const Iq4Tab& t) { return (float)t.val[floor
 QS_DEV int iq4_project_index(float al, const Iq4Tab& t) {
     const float v = al == al ? clampf(2.0f * al, -512.0f, 511.0f) : -200.0f;    // -200: index 1
     return t.idx[floor_int(v) & 1023];
+}
+
+// qs of one block of 32 (iq4_xs.py:180-186): byte j holds the indices of
+// values j and j + 16, so a lane packs its own block in registers
+QS_DEV void iq4_pack(const float (&x)[32], float id, const Iq4Tab& t, uint32_t (&w)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        uint32_t lo = 0, hi = 0;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            lo |= (uint32_t)iq4_project_index(id * x[4 * k + b], t) << (8 * b);
+            hi |= (uint32_t)iq4_project_index(id * x[4 * k + b + 16], t) << (8 * b);
+        }
+        w[k] = lo | (hi << 4);
+    }
 }
 
 // _search_scales_eager iq4_xs.py:52-76 for one block of 32. The two sums of

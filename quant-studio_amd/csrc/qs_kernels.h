@@ -783,32 +783,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const float lsf = clampf(rintf(idq * scale), -32.0f, 31.0f);
     const float dl = d * lsf;
     const float idl = dl != 0.0f ? 1.0f / dl : 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; i++) s.L[slot][32 * g + i] = (uint8_t)iq4_project_index(idl * x[i], iq4tab);
-    s.ls[slot][g] = (int)(lsf + 32.0f);
-    if (g == 0) s.hdr[slot][0] = __builtin_bit_cast(float, f16_bits(d));
+    const int ls = (int)(lsf + 32.0f);
+    s.ls[slot][g] = ls;
     wave_sync();
 
-    const uint8_t* L = s.L[slot];
-    const int* LS = s.ls[slot];
+    // pack (iq4_xs.py:180-186); the staging is 8-byte aligned
     uint8_t* o = s.out + slot * BYTES;
-    const uint32_t dbits = __builtin_bit_cast(uint32_t, s.hdr[slot][0]);
-    for (int bi = g; bi < BYTES; bi += LPS) {
-        uint32_t v;
-        if (bi < 2) v = dbits >> (8 * bi);
-        else if (bi < 4) {
-            uint32_t hb = 0;
+    uint32_t q[4];
+    iq4_pack(x, idl, iq4tab, q);
+    uint64_t* oq = reinterpret_cast<uint64_t*>(o + 8 + 16 * g);
+    oq[0] = q[0] | ((uint64_t)q[1] << 32);
+    oq[1] = q[2] | ((uint64_t)q[3] << 32);
+    const int* LS = s.ls[slot];
+    if (g < 4) o[4 + g] = (uint8_t)((LS[2 * g] & 15) | ((LS[2 * g + 1] & 15) << 4));
+    if (g == 0) {
+        uint32_t h = 0;
 #pragma unroll
-            for (int b = 0; b < 8; b++) hb |= (uint32_t)(LS[b] >> 4) << (2 * b);
-            v = hb >> (8 * (bi - 2));
-        } else if (bi < 8) {
-            const int j = bi - 4;
-            v = (LS[2 * j] & 15) | ((LS[2 * j + 1] & 15) << 4);
-        } else {
-            const int t = bi - 8, blk = t >> 4, j = t & 15;
-            v = L[32 * blk + j] | (L[32 * blk + 16 + j] << 4);
-        }
-        o[bi] = (uint8_t)v;
+        for (int b = 0; b < 8; b++) h |= (uint32_t)(LS[b] >> 4) << (2 * b);
+        *reinterpret_cast<uint32_t*>(o) = f16_bits(d) | (h << 16);
     }
     wave_sync();
     sb_store(s, a);
@@ -849,14 +841,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const float id = scale != 0.0f ? 1.0f / scale : 0.0f;
     uint8_t* o = stage + lane * BYTES;
     const uint32_t h = f16_bits(scale);
-    o[0] = (uint8_t)h;
-    o[1] = (uint8_t)(h >> 8);
+    *reinterpret_cast<uint16_t*>(o) = (uint16_t)h;
+    uint32_t q[4];
+    iq4_pack(x, id, iq4tab, q);
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const int lo = iq4_project_index(id * x[j], iq4tab);
-        const int hi = iq4_project_index(id * x[j + 16], iq4tab);
-        o[2 + j] = (uint8_t)(lo | (hi << 4));
-    }
+    for (int k = 0; k < 4; k++) store_u16x2(o + 2 + 4 * k, q[k]);
     wave_sync();
     const int64_t nvalid = min((int64_t)64, a.n_units - b0);
     const int nbytes = (int)nvalid * BYTES;
