@@ -27,6 +27,7 @@ constexpr float F32_TINY = 1.17549435e-38f;
 
 // native 4 x u32 vector (nontemporal loads need a builtin vector type)
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // Streaming 16-byte load: the source is read exactly once, so it is fetched
 // non-temporally and does not push the kernels' constant tables (imatrix,
@@ -269,12 +270,21 @@ QS_DEV uint32_t f16_bits(float v) {
 QS_DEV float f16_round(float v) { return (float)(_Float16)v; }
 
 // Load n consecutive source elements starting at element offset `off` and
-// widen them to f32 (exact for f16 and bf16). VEC: 16-byte aligned vector loads.
+// widen them to f32 (exact for f16 and bf16). VEC: 16-byte aligned vector loads
+// (one 8-byte load for four 16-bit elements).
 template <int SRC, bool VEC, int N>
 QS_DEV void load_elems(const void* base, int64_t off, float (&out)[N]) {
     if constexpr (SRC == SRC_BF16) {
         const uint16_t* p = static_cast<const uint16_t*>(base) + off;
-        if constexpr (VEC) {
+        if constexpr (VEC && N == 4) {
+            const u32x2 u = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
+            const uint32_t v[2] = {u.x, u.y};
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                out[2 * t] = __builtin_bit_cast(float, v[t] << 16);
+                out[2 * t + 1] = __builtin_bit_cast(float, v[t] & 0xffff0000u);
+            }
+        } else if constexpr (VEC) {
 #pragma unroll
             for (int j = 0; j < N / 8; j++) {
                 const u32x4 u = load_stream16(p + 8 * j);
@@ -291,7 +301,15 @@ QS_DEV void load_elems(const void* base, int64_t off, float (&out)[N]) {
         }
     } else if constexpr (SRC == SRC_F16) {
         const uint16_t* p = static_cast<const uint16_t*>(base) + off;
-        if constexpr (VEC) {
+        if constexpr (VEC && N == 4) {
+            const u32x2 u = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
+            const uint32_t v[2] = {u.x, u.y};
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                out[2 * t] = (float)__builtin_bit_cast(_Float16, (uint16_t)(v[t] & 0xffffu));
+                out[2 * t + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(v[t] >> 16));
+            }
+        } else if constexpr (VEC) {
 #pragma unroll
             for (int j = 0; j < N / 8; j++) {
                 const u32x4 u = load_stream16(p + 8 * j);
@@ -331,7 +349,8 @@ QS_DEV void load_elems(const void* base, int64_t off, float (&out)[N]) {
 // adjacent-pair tree (kq_common.py:38-43); N a power of two
 template <int N>
 QS_DEV float tree_sum(const float (&v)[N]) {
-    float t[N / 2];
+    if constexpr (N == 1) return v[0];
+    float t[(N + 1) / 2];
 #pragma unroll
     for (int i = 0; i < N / 2; i++) t[i] = v[2 * i] + v[2 * i + 1];
 #pragma unroll

@@ -40,7 +40,12 @@ struct QkxResult {
 // 1,797 with five `/` -> 1,395 with shared reciprocals -> 1,269 with the issue
 // breaks (525 instructions at the paired rate would take 1,120); N = 16 871 ->
 // 789 -> 689.
-template <int N, bool MAD>
+//
+// LPG lanes per group (N values each): for shapes with few groups, where a wave's
+// own latency is the time (the launches' rule has the figures). Every lane of
+// the group holds the same sums, so takes the same decisions; all of them must
+// call it.
+template <int N, bool MAD, int LPG = 1>
 QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& steps, float fmax) {
     float mn = x[0], mx = x[0];
 #pragma unroll
@@ -48,13 +53,15 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
         mn = fminf(mn, x[i]);
         mx = fmaxf(mx, x[i]);
     }
+    mn = group_reduce<LPG>(mn, [](float u, float v) { return fminf(u, v); });
+    mx = group_reduce<LPG>(mx, [](float u, float v) { return fmaxf(u, v); });
     mn = fminf(mn, 0.0f);
     const bool degen = (mx == mn);
     float t[N];
-    const float sum_w = tree_sum(w);
+    const float sum_w = group_sum<LPG>(tree_sum(w));
 #pragma unroll
     for (int i = 0; i < N; i++) t[i] = w[i] * x[i];
-    const float sum_x = tree_sum(t);
+    const float sum_x = group_sum<LPG>(tree_sum(t));
 
     float den = degen ? 1.0f : mx - mn;
     const float iscale = fmax / den;
@@ -70,7 +77,8 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
     }
     // a group with mx == mn accepts nothing (its D is 0 or NaN, and no error is
     // below -inf)
-    float best = degen ? -__builtin_inff() : tree_sum(t);
+    float best = group_sum<LPG>(tree_sum(t));
+    best = degen ? -__builtin_inff() : best;
 
     // A range mx - mn, a scale or a min within [LO, HI] and D within [DLO, DHI]
     // keep every division in quotient()'s range: the numerators of scale and min
@@ -83,7 +91,7 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
     // 16-value groups load each step one candidate ahead, so the scalar
     // load's latency is not waited for at the top of every candidate (Q2_K
     // 2-6% faster)
-    constexpr bool AHEAD = N == 16;
+    constexpr bool AHEAD = N <= 16;
     float step_next = steps.v[0];
 #pragma unroll 1
     for (int s = 0; s < steps.n; s++) {
@@ -94,14 +102,14 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
         // the three tree sums are formed 8 values at a time (the tree over N
         // is the trees over its 8-value blocks, then the tree over the block
         // sums), so only one block of products is live at once
-        constexpr int NB = N / 8;
+        constexpr int B = N < 8 ? N : 8, NB = N / B;
         float La[N], sa[NB], sb[NB], sc[NB];
 #pragma unroll
         for (int k = 0; k < NB; k++) {
-            float a[8], b[8], c[8];
+            float a[B], b[B], c[B];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int i = 8 * k + j;
+            for (int j = 0; j < B; j++) {
+                const int i = B * k + j;
                 La[i] = clampf(rintf(isc * (x[i] - mn)), 0.0f, fmax);
                 a[j] = w[i] * La[i];
                 b[j] = a[j] * La[i];
@@ -113,7 +121,8 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
             sc[k] = tree_sum(c);
             issue_break(sc[k]);
         }
-        const float sum_l = tree_sum(sa), sum_l2 = tree_sum(sb), sum_xl = tree_sum(sc);
+        const float sum_l = group_sum<LPG>(tree_sum(sa)), sum_l2 = group_sum<LPG>(tree_sum(sb)),
+                    sum_xl = group_sum<LPG>(tree_sum(sc));
         const float D = sum_w * sum_l2 - sum_l * sum_l;
         const float Dsafe = D > 0 ? D : 1.0f;
         const float num_s = sum_w * sum_xl - sum_x * sum_l, num_m = sum_l2 * sum_x - sum_l * sum_xl;
@@ -142,10 +151,10 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
         float se[NB];
 #pragma unroll
         for (int k = 0; k < NB; k++) {
-            float e8[8];
+            float e8[B];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int i = 8 * k + j;
+            for (int j = 0; j < B; j++) {
+                const int i = B * k + j;
                 float d = this_scale * La[i];
                 d = d + this_min;
                 d = d - x[i];
@@ -155,7 +164,7 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
             se[k] = tree_sum(e8);
             issue_break(se[k]);
         }
-        const float cur = tree_sum(se);
+        const float cur = group_sum<LPG>(tree_sum(se));
         const bool accept = live && cur < best;
         const uint64_t acc = wave_mask(accept);
         far = (far & ~acc) | (wave_mask(out) & acc);
@@ -208,20 +217,24 @@ QS_DEV void quotient_levels(const float (&t)[N], float d, float lo, float hi, fl
 }
 
 // N levels (integers 0 .. 255) as bytes to N consecutive bytes of LDS at a
-// 16-byte boundary: one conversion and merge per value, 16-byte stores (one
+// boundary of min(N, 16) bytes: one conversion and merge per value, 16-byte stores (one
 // byte store per value took a quarter of the requantization)
 template <int N>
 QS_DEV void store_levels(const float (&v)[N], uint8_t* o) {
+    uint32_t w[N / 4];
 #pragma unroll
-    for (int q = 0; q < N / 16; q++) {
-        uint32_t w[4];
+    for (int j = 0; j < N / 4; j++) {
+        w[j] = 0;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            w[j] = 0;
+        for (int b = 0; b < 4; b++) w[j] = __builtin_amdgcn_cvt_pk_u8_f32(v[4 * j + b], b, w[j]);
+    }
+    if constexpr (N >= 16) {
 #pragma unroll
-            for (int b = 0; b < 4; b++) w[j] = __builtin_amdgcn_cvt_pk_u8_f32(v[16 * q + 4 * j + b], b, w[j]);
-        }
-        reinterpret_cast<u32x4*>(o)[q] = u32x4{w[0], w[1], w[2], w[3]};
+        for (int q = 0; q < N / 16; q++)
+            reinterpret_cast<u32x4*>(o)[q] = u32x4{w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]};
+    } else {
+#pragma unroll
+        for (int j = 0; j < N / 4; j++) reinterpret_cast<uint32_t*>(o)[j] = w[j];
     }
 }
 
@@ -333,7 +346,7 @@ QS_DEV float qp_fit(const float (&x)[N], const float (&w)[N], int nmax, const fl
 template <int N, int P, bool WL = false>
 QS_DEV float qp_fit_spread(const float (&x)[N], const float (&w)[N], int nmax, const float (&steps)[8],
                            float (&L)[N], int c, float* xch) {
-    static_assert(P >= 1 && P <= 9, "one to nine lanes share the trials");
+    static_assert(P >= 1, "lanes past the ninth hold no trial");
     const float fmax = (float)nmax;
     const float mx = qp_max(x);
     const bool dead = mx < GROUP_MAX_EPS;

@@ -51,22 +51,6 @@ constexpr int Q40_TILE = 64;                   // blocks per 256-thread tile (4 
 constexpr int Q40_TILES = 4;                   // tiles per workgroup, loaded before any compute
 constexpr int Q40_BLOCKS_PER_WG = Q40_TILE * Q40_TILES;
 
-// Lane (lane ^ M) of the lane's group of four (M = 1 or 2): a DPP quad
-// permute, a VALU move with no LDS round trip (a width-4 __shfl_xor compiles
-// to ds_bpermute and a wait on LDS). Every lane of the group must be active.
-template <int M>
-QS_DEV uint32_t quad_xor(uint32_t v) {
-    static_assert(M == 1 || M == 2, "quad lanes");
-    constexpr int ctrl = M == 1 ? 0xB1 : 0x4E;     // quad_perm:[1,0,3,2] / [2,3,0,1]
-    // bound_ctrl: a quad permute never reads outside the row, so no lane keeps
-    // the (unused) old value
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
-}
-template <int M>
-QS_DEV float quad_xor(float v) {
-    return __builtin_bit_cast(float, quad_xor<M>(__builtin_bit_cast(uint32_t, v)));
-}
-
 // Magnitude of v as an ordered key: the float order for finite and infinite
 // values, every NaN one above Inf and equal to every other NaN, so the first
 // NaN of a block is its maximum, as torch's argmax of |x| takes it
@@ -318,6 +302,24 @@ QS_DEV void sb_store(const SbLds<SPW, BYTES, VSB>& s, const KArgs& a) {
     store_staged(s.out, a.dst, first * BYTES, (int)nvalid * BYTES);
 }
 
+// cascade8_sum over the group of the lane (LPG lanes of V values each), in
+// every one of its lanes. With LPG > 1 the values go through the superblock's
+// 256-value staging; every lane of the wave must call it.
+template <int LPG, int V>
+QS_DEV float group_cascade8(const float (&v)[V], float* stage, int gl) {
+    if constexpr (LPG == 1) {
+        return cascade8_sum(v);
+    } else {
+        constexpr int N = V * LPG;
+        wave_sync();                              // the staging's last readers are done
+#pragma unroll
+        for (int i = 0; i < V; i++) stage[V * gl + i] = v[i];
+        wave_sync();
+        const float* t = stage + N * (gl / LPG);
+        return cascade8_of<N>([&](int i) { return t[i]; });
+    }
+}
+
 // sb_cascade8_256 of x^2 over each superblock of the wave, staged half the
 // wave's superblocks at a time (half the LDS). Every lane takes part in both
 // rounds, the wave barriers included; lanes of the other half compute the
@@ -346,52 +348,54 @@ QS_DEV float sb_sumsq_halves(float (*v)[QK_K], float (*tmp)[40], const float (&x
 // ------------------------------------------------------------------
 // Q4_K / Q5_K  (q4_k.py:25-79, q5_k.py:25-82)
 // ------------------------------------------------------------------
-template <int SRC, bool IMAT, int NMAX, int SQ>
+template <int SRC, bool IMAT, int NMAX, int SQ, int LPG>
 // SQ: the host whose square-root rounding the weights take (SQ_*).
 // Occupancy: 3 waves per SIMD for both variants (135-166 VGPRs). The loop
 // issues at the paired rate from 2 waves up, so the variant without imatrix
 // is no longer held to 128 registers for a fourth wave (12 spilled: 82.6 us for
 // Q5_K f16 2560x4096, 67.3 us at 3 waves).
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_q45_k(KArgs a, Steps steps, QpSteps qps) {
-    constexpr int LPS = 8, SPW = 8, BYTES = NMAX == 15 ? 144 : 176;
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 1 ? 3 : 4))) void k_q45_k(KArgs a, Steps steps, QpSteps qps) {
+    constexpr int LPS = 8 * LPG, SPW = 64 / LPS, V = 32 / LPG, BYTES = NMAX == 15 ? 144 : 176;
     constexpr float FMAX = (float)NMAX;
-    // the imatrix path stages x^2 of all 8 superblocks for sigma2; the other
-    // keeps no per-value staging (its weights need only the lane's own sum)
-    __shared__ SbLds<SPW, BYTES, IMAT ? SPW : 1> s;
-    const SbPos p = sb_pos<LPS, 32>(a.n_units, a.units_per_row, a.stride);
-    const int slot = p.slot, g = p.g;
-    float x[32], w[32];
-    load_elems<SRC, true, 32>(a.src, p.elem, x);
+    // the imatrix path stages x^2 of all the wave's superblocks for sigma2; the
+    // other keeps no per-value staging while a lane holds its whole group (its
+    // weights need only the lane's own sum)
+    __shared__ SbLds<SPW, BYTES, (IMAT || LPG > 1) ? SPW : 1> s;
+    const SbPos p = sb_pos<LPS, V>(a.n_units, a.units_per_row, a.stride);
+    const int slot = p.slot, gl = p.g, g = gl / LPG;       // superblock, lane in it, its group
+    float x[V], w[V];
+    load_elems<SRC, true, V>(a.src, p.elem, x);
 
     if constexpr (IMAT) {
 #pragma unroll
-        for (int i = 0; i < 32; i++) s.v[slot][32 * g + i] = x[i] * x[i];
+        for (int i = 0; i < V; i++) s.v[slot][V * gl + i] = x[i] * x[i];
         wave_sync();
-        const float sum = sb_cascade8_256<LPS>(s.v[slot], s.tmp[slot], g);
+        const float sum = sb_cascade8_256<LPS>(s.v[slot], s.tmp[slot], gl);
         const float sigma2 = (2.0f * sum) / 256.0f;
-        imatrix_weights<32, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
+        imatrix_weights<V, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
     } else {
-        float t[32];
+        float t[V];
 #pragma unroll
-        for (int i = 0; i < 32; i++) t[i] = x[i] * x[i];
-        const float av = sqrt_ref<SQ>(cascade8_sum(t) / 32.0f, a.sqrt);
+        for (int i = 0; i < V; i++) t[i] = x[i] * x[i];
+        const float av = sqrt_ref<SQ>(group_cascade8<LPG>(t, s.v[slot], gl) / 32.0f, a.sqrt);
 #pragma unroll
-        for (int i = 0; i < 32; i++) w[i] = av + fabsf(x[i]);
+        for (int i = 0; i < V; i++) w[i] = av + fabsf(x[i]);
     }
 
-    const QkxResult r = qkx_fit<32, false>(x, w, steps, FMAX);
+    const QkxResult r = qkx_fit<V, false, LPG>(x, w, steps, FMAX);
     s.sc[slot][g] = r.scale;
     s.mn[slot][g] = r.the_min;
-    if constexpr (IMAT) s.sw[slot][g] = cascade8_sum(w);
+    if constexpr (IMAT) s.sw[slot][g] = group_cascade8<LPG>(w, s.v[slot], gl);
     wave_sync();
 
     int ls, lm;
     float d16, m16;
     if constexpr (IMAT) {
-        // make_qp over the 8 scales (lanes 0-3 of the superblock) and the 8
-        // mins (lanes 4-7), each fit's trials spread over its four lanes;
-        // the exchange reuses the sigma2 scratch
-        const int f = g >> 2, c = g & 3;
+        // make_qp over the 8 scales (the lower half of the superblock's lanes)
+        // and the 8 mins (the upper half), each fit's trials spread over its
+        // half; the exchange reuses the sigma2 scratch
+        constexpr int P = LPS / 2;
+        const int f = gl / P, c = gl % P;
         {
             float xv[8], wv[8], L[8];
 #pragma unroll
@@ -399,7 +403,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 xv[i] = f == 0 ? s.sc[slot][i] : s.mn[slot][i];
                 wv[i] = s.sw[slot][i];
             }
-            const float sc = qp_fit_spread<8, 4>(xv, wv, 63, qps.v, L, c, s.tmp[slot] + 18 * f);
+            const float sc = qp_fit_spread<8, P>(xv, wv, 63, qps.v, L, c, s.tmp[slot] + 18 * f);
             if (c == 0) {
                 s.hdr[slot][f] = sc;
 #pragma unroll
@@ -436,15 +440,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 
     const float dg = d16 * (float)(ls & 63), mg = m16 * (float)(lm & 63);
     {
-        float t[32], v[32];
+        float t[V], v[V];
 #pragma unroll
-        for (int i = 0; i < 32; i++) t[i] = x[i] + mg;
+        for (int i = 0; i < V; i++) t[i] = x[i] + mg;
         quotient_levels(t, dg, 0.0f, FMAX, v);
         if (wave_any(dg == 0.0f)) {
 #pragma unroll
-            for (int i = 0; i < 32; i++) v[i] = dg == 0.0f ? qkx_level(r, x[i], FMAX) : v[i];
+            for (int i = 0; i < V; i++) v[i] = dg == 0.0f ? qkx_level(r, x[i], FMAX) : v[i];
         }
-        store_levels(v, s.L[slot] + 32 * g);
+        store_levels(v, s.L[slot] + V * gl);
     }
     wave_sync();
 
@@ -454,21 +458,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const int* LM = s.lm[slot];
     uint8_t* o = s.out + slot * BYTES;
     uint32_t* o4 = reinterpret_cast<uint32_t*>(o);       // BYTES and the staging are multiples of 16
-    if (g == 0) o4[0] = f16_bits(d16) | (f16_bits(m16) << 16);
-    if (g < 4) {
-        o[4 + g] = (uint8_t)(LS[g] | ((LS[4 + g] >> 4) << 6));
-        o[8 + g] = (uint8_t)(LM[g] | ((LM[4 + g] >> 4) << 6));
-        o[12 + g] = (uint8_t)((LS[4 + g] & 15) | ((LM[4 + g] & 15) << 4));
+    if (gl == 0) o4[0] = f16_bits(d16) | (f16_bits(m16) << 16);
+    if (gl < 4) {
+        o[4 + gl] = (uint8_t)(LS[gl] | ((LS[4 + gl] >> 4) << 6));
+        o[8 + gl] = (uint8_t)(LM[gl] | ((LM[4 + gl] >> 4) << 6));
+        o[12 + gl] = (uint8_t)((LS[4 + gl] & 15) | ((LM[4 + gl] & 15) << 4));
     }
-    if constexpr (NMAX == 31) {
-        uint32_t h = 0;                                   // qh: bit 4 of the level of sub-block sb at bit sb
+    if (LPG == 1 || gl < 8) {
+        if constexpr (NMAX == 31) {
+            uint32_t h = 0;                               // qh: bit 4 of the level of sub-block sb at bit sb
 #pragma unroll
-        for (int sb = 0; sb < 8; sb++) h |= ((L[8 * sb + g] >> 4) & 0x01010101u) << sb;
-        o4[4 + g] = h;
-    }
-    {
-        // lane g: 16 bytes of qs, the low nibbles of 16 levels of sub-block 2j and of 2j + 1
-        const int j = g >> 1, l = 4 * (g & 1);
+            for (int sb = 0; sb < 8; sb++) h |= ((L[8 * sb + gl] >> 4) & 0x01010101u) << sb;
+            o4[4 + gl] = h;
+        }
+        // 16 bytes of qs: the low nibbles of 16 levels of sub-block 2j and of 2j + 1
+        const int j = gl >> 1, l = 4 * (gl & 1);
         const u32x4 lo = *reinterpret_cast<const u32x4*>(L + 16 * j + l);
         const u32x4 hi = *reinterpret_cast<const u32x4*>(L + 16 * j + 8 + l);
         *reinterpret_cast<u32x4*>(o4 + (NMAX == 31 ? 12 : 4) + 8 * j + l) =
@@ -648,22 +652,22 @@ __global__ __launch_bounds__(64) void k_q3_k(KArgs a, Steps steps4, Steps steps3
 // ------------------------------------------------------------------
 // Q2_K  (q2_k.py:25-81)
 // ------------------------------------------------------------------
-template <int SRC, bool IMAT, int SQ>
+template <int SRC, bool IMAT, int SQ, int LPG>
 __global__ __launch_bounds__(64) void k_q2_k(KArgs a, Steps steps, QpSteps qps) {
-    constexpr int LPS = 16, SPW = 4, BYTES = 84;
+    constexpr int LPS = 16 * LPG, SPW = 64 / LPS, V = 16 / LPG, BYTES = 84;
     __shared__ SbLds<SPW, BYTES> s;
-    const SbPos p = sb_pos<LPS, 16>(a.n_units, a.units_per_row, a.stride);
-    const int slot = p.slot, g = p.g;
-    float x[16], w[16];
-    load_elems<SRC, true, 16>(a.src, p.elem, x);
+    const SbPos p = sb_pos<LPS, V>(a.n_units, a.units_per_row, a.stride);
+    const int slot = p.slot, gl = p.g, g = gl / LPG;       // superblock, lane in it, its group
+    float x[V], w[V];
+    load_elems<SRC, true, V>(a.src, p.elem, x);
 
     QkxResult r;
     int ls, lm;
     float d16, m16;
     if constexpr (!IMAT) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) w[i] = fabsf(x[i]);
-        r = qkx_fit<16, true>(x, w, steps, 3.0f);
+        for (int i = 0; i < V; i++) w[i] = fabsf(x[i]);
+        r = qkx_fit<V, true, LPG>(x, w, steps, 3.0f);
         s.sc[slot][g] = r.scale;
         s.mn[slot][g] = r.the_min;
         wave_sync();
@@ -682,26 +686,27 @@ __global__ __launch_bounds__(64) void k_q2_k(KArgs a, Steps steps, QpSteps qps) 
         m16 = f16_round(pos_m ? mm / 15.0f : 0.0f);
     } else {
 #pragma unroll
-        for (int i = 0; i < 16; i++) s.v[slot][16 * g + i] = x[i] * x[i];
+        for (int i = 0; i < V; i++) s.v[slot][V * gl + i] = x[i] * x[i];
         wave_sync();
-        const float sigma2 = sb_cascade8_256<LPS>(s.v[slot], s.tmp[slot], g) / 256.0f;
-        imatrix_weights<16, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
-        r = qkx_fit<16, false>(x, w, steps, 3.0f);
+        const float sigma2 = sb_cascade8_256<LPS>(s.v[slot], s.tmp[slot], gl) / 256.0f;
+        imatrix_weights<V, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
+        r = qkx_fit<V, false, LPG>(x, w, steps, 3.0f);
         s.sc[slot][g] = r.scale;
         s.mn[slot][g] = r.the_min;
-        s.sw[slot][g] = cascade8_sum(w);
+        s.sw[slot][g] = group_cascade8<LPG>(w, s.v[slot], gl);
         wave_sync();
         {
-            // the 16 scales on lanes 0-7 of the superblock, the 16 mins on
-            // lanes 8-15, each fit's trials spread over its eight lanes
-            const int f = g >> 3, c = g & 7;
+            // the 16 scales on the lower half of the superblock's lanes, the 16
+            // mins on the upper half, each fit's trials spread over its half
+            constexpr int P = LPS / 2;
+            const int f = gl / P, c = gl % P;
             float xv[16], wv[16], L[16];
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 xv[i] = f == 0 ? s.sc[slot][i] : s.mn[slot][i];
                 wv[i] = s.sw[slot][i];
             }
-            const float sc = qp_fit_spread<16, 8>(xv, wv, 15, qps.v, L, c, s.tmp[slot] + 18 * f);
+            const float sc = qp_fit_spread<16, P>(xv, wv, 15, qps.v, L, c, s.tmp[slot] + 18 * f);
             if (c == 0) {
                 s.hdr[slot][f] = sc;
 #pragma unroll
@@ -721,28 +726,30 @@ __global__ __launch_bounds__(64) void k_q2_k(KArgs a, Steps steps, QpSteps qps) 
     const int scb = (ls | (lm << 4)) & 0xFF;
     const float dg = d16 * (float)(scb & 15), mg = m16 * (float)(scb >> 4);
     {
-        float t[16], v[16];
+        float t[V], v[V];
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = x[i] + mg;
+        for (int i = 0; i < V; i++) t[i] = x[i] + mg;
         quotient_levels(t, dg, 0.0f, 3.0f, v);
         if (wave_any(dg == 0.0f)) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) v[i] = dg == 0.0f ? qkx_level(r, x[i], 3.0f) : v[i];
+            for (int i = 0; i < V; i++) v[i] = dg == 0.0f ? qkx_level(r, x[i], 3.0f) : v[i];
         }
-        store_levels(v, s.L[slot] + 16 * g);
+        store_levels(v, s.L[slot] + V * gl);
     }
     wave_sync();
 
     // pack (q2_k.py:74-80), a word of four levels at a time
     uint8_t* o = s.out + slot * BYTES;
     uint32_t* o4 = reinterpret_cast<uint32_t*>(o);        // BYTES is a multiple of 4
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(s.L[slot]) + 32 * (g >> 3) + (g & 7);
-    uint32_t v = 0;                                       // qs bytes 4 g .. + 3
+    if (LPG == 1 || gl < 16) {
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(s.L[slot]) + 32 * (gl >> 3) + (gl & 7);
+        uint32_t v = 0;                                   // qs bytes 4 gl .. + 3
 #pragma unroll
-    for (int i = 0; i < 4; i++) v |= q[8 * i] << (2 * i);
-    o4[4 + g] = v;
+        for (int i = 0; i < 4; i++) v |= q[8 * i] << (2 * i);
+        o4[4 + gl] = v;
+    }
     o[g] = (uint8_t)scb;
-    if (g == 0) o4[20] = f16_bits(d16) | (f16_bits(m16) << 16);
+    if (gl == 0) o4[20] = f16_bits(d16) | (f16_bits(m16) << 16);
     wave_sync();
     sb_store(s, a);
 }

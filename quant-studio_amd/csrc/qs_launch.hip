@@ -82,6 +82,44 @@ hipError_t launch_b32(const qs::KArgs& a, hipStream_t st) {
     return launch(qs::k_b32<SRC, T>, dim3(g), dim3(256), st, a);
 }
 
+// One wave per workgroup of 64 / lps superblocks
+dim3 sb_grid(const qs::KArgs& a, int lps) { return dim3((unsigned)((a.n_units + 64 / lps - 1) / (64 / lps))); }
+
+// Lanes per group of the make_qkx kernels. A launch of a wave or two per SIMD
+// (256 CUs x 4) takes as long as one wave, whose time is its instruction
+// count: splitting a group over 8 (Q2_K: 4) lanes cuts that to about 0.4 for 2.1
+// times the work, over 4 lanes to 0.5 for 1.5 times. So 8 lanes while that
+// makes at most 2 waves per SIMD (2,048 superblocks), 4 while it makes at most
+// 3 (6,144). Measured, k = 2560, us at 1 / 4 / 8 lanes per group:
+//   Q4_K imatrix  160 superblocks 55.0 / 26.2 / 22.0, 2,040 54.9 / 27.9 / 26.2,
+//                 4,100 57.0 / 40.8 / 45.5, 8,200 60.6 / 59.3 / 72.1
+//   Q4_K          160 29.6 / 14.3 / 12.2, 2,040 29.7 / 15.8 / 15.3,
+//                 4,100 30.4 / 23.3 / 26.1, 8,200 33.1 / 34.2 / 41.0
+//   Q5_K          160 23.7 / 11.8 / 10.6, 2,040 23.8 / 13.1 / 12.8,
+//                 4,100 24.5 / 19.1 / 21.4, 8,200 26.5 / 28.2 / 33.4
+// and Q2_K at 1 / 2 / 4 lanes (2 lanes are never ahead by 5%):
+//   with imatrix  160 38.6 / 29.1 / 24.3, 2,040 40.7 / 31.0 / 29.6, 4,100 41.5 / 43.1 / 47.0
+//   without       160 15.0 / 11.9 / 11.6, 2,040 16.0 / 12.6 / 11.9, 4,100 16.9 / 17.6 / 19.9
+constexpr int64_t kSplit8 = 2048, kSplit4 = 6144;
+
+template <int SRC, bool IMAT, int NMAX, int SQ>
+hipError_t launch_q45(const qs::KArgs& a, hipStream_t st, const qs::Steps& steps) {
+    const dim3 wave(64);
+    if (a.n_units <= kSplit8)
+        return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 8>, sb_grid(a, 64), wave, st, a, steps, qp_steps(63));
+    if (a.n_units <= kSplit4)
+        return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 4>, sb_grid(a, 32), wave, st, a, steps, qp_steps(63));
+    return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 1>, sb_grid(a, 8), wave, st, a, steps, qp_steps(63));
+}
+
+template <int SRC, bool IMAT, int SQ>
+hipError_t launch_q2(const qs::KArgs& a, hipStream_t st, const qs::Steps& steps) {
+    const dim3 wave(64);
+    if (a.n_units <= kSplit8)
+        return launch(qs::k_q2_k<SRC, IMAT, SQ, 4>, sb_grid(a, 64), wave, st, a, steps, qp_steps(15));
+    return launch(qs::k_q2_k<SRC, IMAT, SQ, 1>, sb_grid(a, 16), wave, st, a, steps, qp_steps(15));
+}
+
 // SQ: the host whose square-root rounding the weights take (qs::SQ_*);
 // kernels whose weights take no square root are instantiated once (SQ_IEEE).
 template <int SRC, int SQ>
@@ -102,15 +140,11 @@ hipError_t launch_type(int type, bool imat, const qs::KArgs& a, hipStream_t st,
                     : launch(k_iq4_nl<SRC, false, SQ_IEEE>, g, wave, st, a);
     }
     case QS_TYPE_Q4_K:
-        return imat ? launch(k_q45_k<SRC, true, 15, SQ>, sb8, wave, st, a, qkx_steps(-0.9f, 0.05f, 36, 15),
-                             qp_steps(63))
-                    : launch(k_q45_k<SRC, false, 15, SQ>, sb8, wave, st, a, qkx_steps(-1.0f, 0.1f, 20, 15),
-                             qp_steps(63));
+        return imat ? launch_q45<SRC, true, 15, SQ>(a, st, qkx_steps(-0.9f, 0.05f, 36, 15))
+                    : launch_q45<SRC, false, 15, SQ>(a, st, qkx_steps(-1.0f, 0.1f, 20, 15));
     case QS_TYPE_Q5_K:
-        return imat ? launch(k_q45_k<SRC, true, 31, SQ>, sb8, wave, st, a, qkx_steps(-0.9f, 0.05f, 36, 31),
-                             qp_steps(63))
-                    : launch(k_q45_k<SRC, false, 31, SQ>, sb8, wave, st, a, qkx_steps(-0.5f, 0.1f, 15, 31),
-                             qp_steps(63));
+        return imat ? launch_q45<SRC, true, 31, SQ>(a, st, qkx_steps(-0.9f, 0.05f, 36, 31))
+                    : launch_q45<SRC, false, 31, SQ>(a, st, qkx_steps(-0.5f, 0.1f, 15, 31));
     case QS_TYPE_Q6_K:
         return imat ? launch(k_q6_k<SRC, true>, sb4, wave, st, a, qx_steps(32))
                     : launch(k_q6_k<SRC, false>, sb4, wave, st, a, qx_steps(32));
@@ -118,10 +152,8 @@ hipError_t launch_type(int type, bool imat, const qs::KArgs& a, hipStream_t st,
         return imat ? launch(k_q3_k<SRC, true, SQ>, sb4, wave, st, a, qx_steps(4), qx_steps(32))
                     : launch(k_q3_k<SRC, false, SQ_IEEE>, sb4, wave, st, a, qx_steps(4), qx_steps(32));
     case QS_TYPE_Q2_K:
-        return imat ? launch(k_q2_k<SRC, true, SQ>, sb4, wave, st, a, qkx_steps(-0.9f, 0.05f, 36, 3),
-                             qp_steps(15))
-                    : launch(k_q2_k<SRC, false, SQ_IEEE>, sb4, wave, st, a, qkx_steps(-0.5f, 0.1f, 15, 3),
-                             qp_steps(15));
+        return imat ? launch_q2<SRC, true, SQ>(a, st, qkx_steps(-0.9f, 0.05f, 36, 3))
+                    : launch_q2<SRC, false, SQ_IEEE>(a, st, qkx_steps(-0.5f, 0.1f, 15, 3));
     case QS_TYPE_IQ4_XS:
         return imat ? launch(k_iq4_xs<SRC, true, SQ>, sb8, wave, st, a)
                     : launch(k_iq4_xs<SRC, false, SQ_IEEE>, sb8, wave, st, a);

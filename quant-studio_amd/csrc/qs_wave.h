@@ -49,6 +49,42 @@ QS_DEV int wave_incl_scan(int x) {
     return v;
 }
 
+// Lane (lane ^ M) of the lane's group of four (M = 1 or 2): a DPP quad
+// permute, a VALU move with no LDS round trip (a width-4 __shfl_xor compiles
+// to ds_bpermute and a wait on LDS). Every lane of the group must be active.
+template <int M>
+QS_DEV uint32_t quad_xor(uint32_t v) {
+    static_assert(M == 1 || M == 2, "quad lanes");
+    constexpr int ctrl = M == 1 ? 0xB1 : 0x4E;     // quad_perm:[1,0,3,2] / [2,3,0,1]
+    // bound_ctrl: a quad permute never reads outside the row, so no lane keeps
+    // the (unused) old value
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+template <int M>
+QS_DEV float quad_xor(float v) {
+    return __builtin_bit_cast(float, quad_xor<M>(__builtin_bit_cast(uint32_t, v)));
+}
+
+// f over the LPG (1, 2, 4 or 8) consecutive lanes of a group, for an f whose
+// value does not depend on operand order: a butterfly, so every lane ends with
+// the same bits. A sum taken this way continues an adjacent-pair tree: lane q
+// holds the tree over its own consecutive values, each level joins two
+// adjacent subtrees, and fl(a + b) = fl(b + a). The last level of eight lanes
+// reads the mirrored lane of the other quad, whose four lanes hold one value.
+template <int LPG, typename F>
+QS_DEV float group_reduce(float v, F&& f) {
+    static_assert(LPG == 1 || LPG == 2 || LPG == 4 || LPG == 8, "lanes per group");
+    if constexpr (LPG >= 2) v = f(v, quad_xor<1>(v));
+    if constexpr (LPG >= 4) v = f(v, quad_xor<2>(v));
+    if constexpr (LPG >= 8)      // row_half_mirror
+        v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true)));
+    return v;
+}
+template <int LPG>
+QS_DEV float group_sum(float v) {
+    return group_reduce<LPG>(v, [](float a, float b) { return a + b; });
+}
+
 // Superblock position of this lane.
 struct SbPos {
     int64_t sb;      // global superblock index (clamped copy used for loads)
@@ -81,14 +117,16 @@ QS_DEV SbPos sb_pos(int64_t n_sb, int64_t sb_per_row, int64_t stride) {
 // `v` is the superblock's 256 values in LDS; `tmp` holds 40 floats.
 template <int LPS, bool WL = false>
 QS_DEV float sb_cascade8_256(const float* v, float* tmp, int g) {
-    constexpr int PER = 32 / LPS;
+    constexpr int PER = LPS < 32 ? 32 / LPS : 1;
+    if (LPS <= 32 || g < 32) {
 #pragma unroll
-    for (int t = 0; t < PER; t++) {
-        const int j = g * PER + t;             // j = 8a + l
-        float acc = 0.0f;
+        for (int t = 0; t < PER; t++) {
+            const int j = g * PER + t;             // j = 8a + l
+            float acc = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) acc = acc + v[32 * i + j];
-        tmp[j] = acc;
+            for (int i = 0; i < 8; i++) acc = acc + v[32 * i + j];
+            tmp[j] = acc;
+        }
     }
     wave_sync<WL>();
     if (g < 8) {

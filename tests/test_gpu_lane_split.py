@@ -1,0 +1,44 @@
+"""Calls of few superblocks take other variants of a kernel than calls of many
+(several lanes per group); their bytes are the same, and the oracle's."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from test_gpu_parity import dev  # noqa: F401 (fixture)
+
+pytestmark = pytest.mark.gpu
+
+# superblocks per call on both sides of every line of the dispatch, and one
+# superblock, and counts that leave a wave partly empty
+COUNTS = [1, 3, 255, 2048, 2049, 6143, 6144]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("imat", [False, True])
+@pytest.mark.parametrize("qtype", ["q2_k", "q4_k", "q5_k"])
+def test_variants_agree_over_the_dispatch(qs, dev, qtype, imat, dtype):  # noqa: F811
+    gen = torch.Generator(device="cuda").manual_seed(17)
+    rows = 8200
+    x = torch.randn(rows, 256, generator=gen, device=dev) * 0.02
+    x *= torch.exp(torch.randn(rows, 1, generator=gen, device=dev))
+    x[5] = 0
+    x[6] = 0.125
+    x[7, :128] = 0
+    x[8, 32:48] = x[8, 32]
+    x[9] = x[9].abs()
+    x[10:12] *= 1e-13
+    x[12:14] *= 1e13 if dtype == torch.float32 else 1e4
+    x[14, 100] = 3.0
+    x = x.to(dtype)
+    qw = torch.exp(torch.randn(256, generator=gen, device=dev)) if imat else None
+    if imat:
+        qw[::7] = 0
+    fn = qs.QUANT_TYPES[qtype].make_kernel(dev, qw)
+    whole = fn(x).cpu()
+    ref = oracle.quantize(qtype, x[:600].float().cpu().numpy(), None if qw is None else qw.cpu().numpy())
+    assert np.array_equal(whole[:600].numpy(), ref)
+    for n in COUNTS:
+        assert torch.equal(fn(x[:n]).cpu(), whole[:n]), n
+        assert torch.equal(fn(x[rows - n:]).cpu(), whole[rows - n:]), n
