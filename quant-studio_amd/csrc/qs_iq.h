@@ -176,8 +176,7 @@ QS_DEV float level(const Levels<NV>& L, int e) {
 // level's |d| is strictly below both neighbouring levels' (the grid's levels
 // are 0..3 for IQ2 and 0..7 for IQ3; at an end the missing neighbour is not
 // needed), d changes sign there, every other level's |d| is at least the
-// code level's, and so is its term: the check takes two instructions a
-// level instead of the four a term takes. The weights are square roots
+// code level's, and so is its term. The weights are square roots
 // (>= 0, -0 or NaN). A NaN weight makes every distance NaN (the first entry
 // wins, and no reduced list leaves it out); at a +inf weight only the code's
 // level can have d = 0, so an entry left out for an earlier one that keeps
@@ -186,60 +185,53 @@ QS_DEV float level(const Levels<NV>& L, int e) {
 // check fails only in values at the clamped top level 2 (IQ2) whose level-3
 // |d| is strictly below the level-2 |d| (so d < 0 at level 2 and levels 0 and
 // 1 have terms no smaller), the clamp-tolerant reduced list is read (an entry
-// it leaves out also shares every raise to level 3 with the earlier one). A
-// NaN or infinite d at the code level, a tie or sc <= 0 reads the full
-// list. PRUNE 0 reads the full lists.
+// it leaves out also shares every raise to level 3 with the earlier one).
+// PRUNE 0 reads the full lists.
+//
+// The check reads the position of the value between the levels instead of
+// forming the three |d|: u = max(t, 0) - level, t = 0.5*(inv*x - 1), is
+// half of x/sc minus the code's odd level, within 2^-18 while it is below 2^10
+// (inv * sc is 1 within an ulp). |u| < 1/2 - 2^-10 puts the code level's |d| at
+// most (1 - 2^-9 + 2^-17) sc, a neighbour's at least (1 + 2^-9 - 2^-17) sc, and
+// the f32 rounding of a d is below 2^-20 sc, so the strict order holds;
+// max(t, 0) drops the lower neighbour of level 0, which does not exist. Past
+// the top level, 1/2 + 2^-10 < u < 2^10 puts the next level's |d| strictly
+// below. In between, and for scales outside 2^+-100, the full list is read. A
+// NaN value counts as u = 0: every distance is then NaN, and the first entry
+// wins in either list. 9 instructions a value, 4 at half rate, for 28 that
+// compared the |d| and packed the code with integer shifts (the code is
+// summed in f32, exact below 2^24).
 template <int BITS, int NV, int NSUB, int PRUNE = 0, int N>
 QS_DEV void iq_codes(const IqTabDev& T, const float (&xv)[N], float inv, uint32_t (&ci)[NSUB], float sc) {
     // all subgroups' codes first, so their cinfo loads are in flight together
     constexpr float LMAX = BITS == 2 ? 2.0f : 7.0f;
-    constexpr float GMAX = BITS == 2 ? 3.0f : 7.0f;     // the grid's largest level
-    // per subgroup, PRUNE 1: whether the code's level is every value's best
-    // level, a bool (a lane mask: its updates take no VALU instructions);
-    // PRUNE 2: an int with bit 0 set when a value's code level is not its
-    // best level and bit 1 when the clamp-tolerant list does not hold either
-    // (two bools per subgroup spill in the IQ2_XXS search)
-    int code[NSUB], miss[NSUB];
-    bool best[NSUB];
-    const bool prune = PRUNE > 0 && sc > 0.0f;
+    constexpr float EPS = 0x1p-10f;
+    const bool prune = PRUNE > 0 && sc >= 0x1p-100f && sc <= 0x1p100f;
+    int code[NSUB];
 #pragma unroll
     for (int s = 0; s < NSUB; s++) {
-        code[s] = 0;
-        best[s] = prune;
-        miss[s] = prune ? 0 : 3;
+        float sum = 0.0f, far = -1.0f, near = 1.0f;     // largest |u| - 1/2, and its smallest magnitude
 #pragma unroll
         for (int j = 0; j < NV; j++) {
-            const float x = xv[NV * s + j];
-            float t = inv * x;
-            t = t - 1.0f;
-            t = 0.5f * t;
-            const float lf = clampf(rintf(t), 0.0f, LMAX);
-            code[s] |= (int)lf << (BITS * j);
+            // 0.5 * fl(p - 1) = fl(0.5 p - 0.5)
+            const float t = fmaxf(__builtin_fmaf(inv * xv[NV * s + j], 0.5f, -0.5f), 0.0f);
+            const float lf = fminf(rintf(t), LMAX);
+            sum = __builtin_fmaf(lf, (float)(1 << (BITS * j)), sum);
             if constexpr (PRUNE > 0) {
-                const float v = 2.0f * lf + 1.0f;
-                auto dist = [&](float lv) {
-                    float d = sc * lv;
-                    d = d - x;
-                    return fabsf(d);
-                };
-                const float du = dist(v), dm = dist(v - 2.0f), dp = dist(v + 2.0f);
-                const bool ok = (lf == 0.0f || du < dm) && (lf == GMAX || du < dp);
-                if constexpr (PRUNE == 2) {
-                    // the clamped top level with the grid's level 3 strictly closer
-                    const bool up = LMAX < GMAX && lf == LMAX && dp < du;
-                    miss[s] |= ok ? 0 : up ? 1 : 3;
-                } else {
-                    best[s] = best[s] && ok;
-                }
+                const float h = fabsf(t - lf) - 0.5f;
+                far = fmaxf(far, h);
+                if constexpr (PRUNE == 2) near = fminf(near, fabsf(h));
             }
+        }
+        code[s] = (int)sum;
+        if constexpr (PRUNE > 0) {
+            int tab = far < -EPS ? 1 : 0;
+            if constexpr (PRUNE == 2) tab = far >= -EPS && far < 0x1p10f && near > EPS ? 2 : tab;
+            code[s] += prune ? tab * T.ncodes : 0;
         }
     }
 #pragma unroll
-    for (int s = 0; s < NSUB; s++) {
-        int tab = best[s] ? 1 : 0;
-        if constexpr (PRUNE == 2) tab = miss[s] == 0 ? 1 : miss[s] == 1 ? 2 : 0;
-        ci[s] = T.cinfo[code[s] + tab * T.ncodes];
-    }
+    for (int s = 0; s < NSUB; s++) ci[s] = T.cinfo[code[s]];
 }
 
 // The values and distance weights of one subgroup, passed by value.
