@@ -379,7 +379,7 @@ bool sqrt_map_bits(int id, const std::vector<uint32_t>*& out) {
     if (id == SQM_INTEL_DOWN) {
         std::call_once(intel_once, [] {
             auto& b = bits[SQM_INTEL_DOWN];
-            b.assign(1u << 19, 0u);
+            b.assign(qs::SQRT_MAP_WORDS, 0u);
             uint32_t key = 0;
             for (int i = 0; i < QS_SQRT_DOWN_N; i++) {
                 key += QS_SQRT_DOWN_GAPS[i];
@@ -389,8 +389,8 @@ bool sqrt_map_bits(int id, const std::vector<uint32_t>*& out) {
         return true;
     }
     std::call_once(amd_once, [] {
-        bits[SQM_AMD_DOWN].assign(1u << 19, 0u);
-        bits[SQM_AMD_UP].assign(1u << 19, 0u);
+        bits[SQM_AMD_DOWN].assign(qs::SQRT_MAP_WORDS, 0u);
+        bits[SQM_AMD_UP].assign(qs::SQRT_MAP_WORDS, 0u);
         std::vector<unsigned char> packed(1u << 22);
         uLongf len = (uLongf)packed.size();
         const uLong clen = (uLong)(qs_sqrt_amd_blob_end - qs_sqrt_amd_blob);

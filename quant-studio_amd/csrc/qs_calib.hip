@@ -86,9 +86,24 @@ __global__ __launch_bounds__(256) void k_recip(int e, uint32_t* worst, uint32_t*
     if (bad) atomicAdd(differ, bad);
 }
 
+// One thread per mantissa of v = m 2^(2 k + parity): the roots that differ from sqrtf
+__global__ __launch_bounds__(256) void k_sqrt(int k, uint32_t* differ) {
+    const uint32_t key = blockIdx.x * 256u + threadIdx.x;           // 2^24 threads
+    const float v = ldexpf(__uint_as_float(0x3f800000u + key), 2 * k);      // [1, 4) 4^k
+    if (__float_as_uint(qs::sqrt_root(v)) != __float_as_uint(sqrtf(v))) atomicAdd(differ, 1u);
+}
+
 }  // namespace
 
 extern "C" {
+
+// Check qs::sqrt_root for every v in [4^k, 4^(k+1)) (k -48 .. 53) on hip_stream;
+// result: a device word, zeroed by the caller.
+int qs_calib_sqrt(int k, unsigned* result, void* hip_stream) {
+    if (!result || k < -48 || k > 53) return -22;
+    hipLaunchKernelGGL(k_sqrt, dim3((1u << 24) / 256), dim3(256), 0, static_cast<hipStream_t>(hip_stream), k, result);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+}
 
 // Check qs::recip and qs::quotient over every mantissa of a divisor of exponent
 // e (-60 .. 60) on hip_stream; result: two device words, zeroed by the caller

@@ -127,6 +127,25 @@ struct SqrtMap {
     const uint32_t* up;
 };
 
+// A map's words: its 2^24 bits, then zero words for lanes that look nothing up
+constexpr uint32_t SQRT_MAP_ZERO = 1u << 19, SQRT_MAP_WORDS = SQRT_MAP_ZERO + 16;
+
+// The IEEE square root of v in [2^-96, 2^108]: v_rsq_f32, one coupled iteration
+// for the root and half its reciprocal, and an exact-remainder correction (P.
+// Markstein, "IA-64 and Elementary Functions", 2000). Compared with sqrtf on
+// the device for every mantissa and exponent parity (qs_calib_sqrt); scaling v
+// by 4^k scales every step exactly. 7 full-rate instructions and the v_rsq_f32
+// for sqrtf's 16, 9 of them at half rate or less.
+QS_DEV float sqrt_root(float v) {
+    float y = __builtin_amdgcn_rsqf(v);
+    issue_break(y);
+    float g = v * y, h = 0.5f * y;
+    const float e = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, e, g);
+    h = __builtin_fmaf(h, e, h);
+    return __builtin_fmaf(__builtin_fmaf(-g, g, v), h, g);
+}
+
 // true for inputs the maps apply to: positive finite (Intel), positive
 // normal finite (AMD)
 template <int SQ>
@@ -236,30 +255,116 @@ QS_DEV void sqrt_ref_n(const float (&v)[N], const SqrtMap& m, float (&out)[N]) {
     }
 }
 
+// sqrt_ref of N values that are normal, positive and within [2^-80, 2^108] (so
+// neither subnormal keys nor the always-read range of sqrt_lookup_key occur),
+// or 0 where ZERO is set; the same band test and map bits, in about 22
+// instructions a value, 4 at half rate, where the general form takes some 45
+// and a branch. A value outside the band reads a zero word, so nothing is
+// masked afterwards.
+template <int N, int SQ, bool ZERO>
+QS_DEV void sqrt_ref_normal(const float (&v)[N], const SqrtMap& m, float (&out)[N]) {
+    uint32_t at[N], wd[N], wu[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        out[i] = sqrt_root(v[i]);
+        if constexpr (SQ != SQ_IEEE) {
+            const float r = out[i];
+            const float rem = __builtin_fmaf(-r, r, v[i]);
+            const float ulp = __uint_as_float((__float_as_uint(r) & 0x7f800000u) - (23u << 23));
+            bool look;
+            if constexpr (SQ == SQ_AMD) {
+                const float lim = (0.48f * r) * ulp;
+                look = fabsf(rem) > lim;
+            } else {
+                look = rem < (-0.875f * r) * ulp;
+            }
+            const uint32_t byte = (__float_as_uint(v[i]) ^ 0x00800000u) >> 3 & 0x001ffffcu;
+            at[i] = look ? byte : 4u * SQRT_MAP_ZERO;
+        }
+    }
+    if constexpr (SQ != SQ_IEEE) {
+        auto word = [](const uint32_t* map, uint32_t at) {
+            return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(map) + at);
+        };
+#pragma unroll
+        for (int i = 0; i < N; i++) wd[i] = word(m.down, at[i]);
+        if constexpr (SQ == SQ_AMD) {
+#pragma unroll
+            for (int i = 0; i < N; i++) wu[i] = word(m.up, at[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t key = __float_as_uint(v[i]);     // its low 5 bits are the map key's
+            uint32_t b = __float_as_uint(out[i]) - __builtin_amdgcn_ubfe(wd[i], key, 1);
+            if constexpr (SQ == SQ_AMD) b += __builtin_amdgcn_ubfe(wu[i], key, 1);
+            out[i] = __uint_as_float(b);
+        }
+    }
+    if constexpr (ZERO) {
+#pragma unroll
+        for (int i = 0; i < N; i++) out[i] = v[i] == 0.0f ? 0.0f : out[i];
+    }
+}
+
+// sqrt_ref_n by sqrt_ref_normal where every value of the wave is +0 or in its range
+template <int N, int SQ>
+QS_DEV void sqrt_ref_wave(const float (&v)[N], const SqrtMap& m, float (&out)[N]) {
+    uint32_t lo = 0xffffffffu, hi = 0;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        lo = min(lo, __float_as_uint(v[i]) - 1u);           // +0 is the largest
+        hi = max(hi, __float_as_uint(v[i]));
+    }
+    const bool in = lo >= 0x17800000u - 1u && hi <= 0x71800000u;      // 2^-80, 2^100
+    constexpr int CH = N < 8 ? N : 8;
+    auto chunks = [&](auto roots) {
+#pragma unroll
+        for (int c = 0; c < N; c += CH) {
+            float t[CH], r[CH];
+#pragma unroll
+            for (int i = 0; i < CH; i++) t[i] = v[c + i];
+            roots(t, r);
+#pragma unroll
+            for (int i = 0; i < CH; i++) {
+                out[c + i] = r[i];
+                keep_in_register(out[c + i]);
+            }
+        }
+    };
+    if (wave_any(!in)) chunks([&](const float (&t)[CH], float (&r)[CH]) { sqrt_ref_n<CH, true, SQ>(t, m, r); });
+    else chunks([&](const float (&t)[CH], float (&r)[CH]) { sqrt_ref_normal<CH, SQ, true>(t, m, r); });
+}
+
 // imatrix weights w[i] = qw[i] * sqrt_ref(sigma2 + x[i]^2) (e.g. q4_k.py:51),
 // with the imatrix and map loads of CH values issued together (CH < N bounds
-// the registers the phase holds, for kernels whose occupancy it would set)
-template <int N, bool BAND, int SQ, int CH = N>
+// the registers the phase holds: whole groups at once spilled 34-84 registers)
+template <int N, bool BAND, int SQ, int CH = (N < 8 ? N : 8)>
 QS_DEV void imatrix_weights(const float* __restrict__ qw, float sigma2, const float (&x)[N],
                             const SqrtMap& m, float (&w)[N]) {
     static_assert(N % CH == 0, "chunks tile the group");
+    // x^2 is at most 256 sigma2 (sigma2 is a mean over at most 256 squares, x's
+    // among them), so sigma2 bounds every root's input
+    const bool general = wave_any(!(sigma2 >= 0x1p-80f && sigma2 <= 0x1p99f));
+    auto weights = [&](auto roots) {
 #pragma unroll
-    for (int c = 0; c < N; c += CH) {
-        float v[CH], q[CH];
+        for (int c = 0; c < N; c += CH) {
+            float v[CH], q[CH], r[CH];
 #pragma unroll
-        for (int i = 0; i < CH; i++) {
-            const float t = x[c + i] * x[c + i];
-            v[i] = sigma2 + t;
-            q[i] = qw[c + i];
+            for (int i = 0; i < CH; i++) {
+                const float t = x[c + i] * x[c + i];
+                v[i] = sigma2 + t;
+                q[i] = qw[c + i];
+            }
+            roots(v, r);
+#pragma unroll
+            for (int i = 0; i < CH; i++) {
+                w[c + i] = q[i] * r[i];
+                if constexpr (CH < N) keep_in_register(w[c + i]);
+            }
         }
-        float r[CH];
-        sqrt_ref_n<CH, BAND, SQ>(v, m, r);
-#pragma unroll
-        for (int i = 0; i < CH; i++) {
-            w[c + i] = q[i] * r[i];
-            if constexpr (CH < N) keep_in_register(w[c + i]);
-        }
-    }
+    };
+    if (general) weights([&](const float (&v)[CH], float (&r)[CH]) { sqrt_ref_n<CH, BAND, SQ>(v, m, r); });
+    else weights([&](const float (&v)[CH], float (&r)[CH]) { sqrt_ref_normal<CH, SQ, false>(v, m, r); });
 }
 
 // f32 -> fp16 bits, round to nearest even (v_cvt_f16_f32 under the default mode)

@@ -607,7 +607,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const int slot = p.slot, g = p.g;
     float x[32], w[32], waux[32], xval[32];
     iq_load_weights<SRC, LPS, 32, SQ>(a, p, s.v, s.tmp, 1.0f, false, x, w);
-    sqrt_ref_n<32, true, SQ>(w, a.sqrt, waux);
+    sqrt_ref_wave<32, SQ>(w, a.sqrt, waux);
     keep_in_registers(waux);
     int signs[4];
     static_for<0, 4>([&](auto S) { signs[S] = parity_fold8<8 * S>(x, w, xval); });
@@ -730,7 +730,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
     const int slot = p.slot, g = p.g;
     float x[16], w[16], waux[16], xval[16];
     iq_load_weights<SRC, LPS, 16, SQ, WL>(a, p, s.v, s.tmp, IS_S ? 2.0f : 1.0f, false, x, w);
-    sqrt_ref_n<16, true, SQ>(w, a.sqrt, waux);
+    sqrt_ref_wave<16, SQ>(w, a.sqrt, waux);
     int signs[2];
     if constexpr (IS_S) {
         signs[0] = sign_bits8<0>(x, xval);
@@ -881,7 +881,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
     const int slot = p.slot, grp = p.g / LPG, q = p.g % LPG;
     float x[VPL], w[VPL], waux[VPL], xval[VPL];
     iq_load_weights<SRC, LPS, VPL, SQ>(a, p, s.v, s.tmp, 2.0f, !IMAT, x, w);
-    sqrt_ref_n<VPL, true, SQ>(w, a.sqrt, waux);
+    sqrt_ref_wave<VPL, SQ>(w, a.sqrt, waux);
     keep_in_registers(waux);
     int signs[NCH];
     if constexpr (IS_S) {

@@ -758,7 +758,7 @@ __global__ __launch_bounds__(64) void k_q2_k(KArgs a, Steps steps, QpSteps qps) 
 // IQ4_XS  (iq4_xs.py:149-188)
 // ------------------------------------------------------------------
 template <int SRC, bool IMAT, int SQ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_iq4_xs(KArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_iq4_xs(KArgs a) {
     constexpr int LPS = 8, SPW = 8, BYTES = 136;
     // LDS is what limits this kernel's residency: the imatrix path stages x^2
     // for sigma2 half the wave's superblocks at a time, the other stages none
@@ -771,7 +771,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     load_elems<SRC, true, 32>(a.src, p.elem, x);
     if constexpr (IMAT) {
         const float sigma2 = (2.0f * sb_sumsq_halves<LPS, SPW, 32>(s.v, s.tmp, x, slot, g)) / 256.0f;
-        imatrix_weights<32, true, SQ, 8>(a.qw + p.col, sigma2, x, a.sqrt, w);
+        imatrix_weights<32, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
     } else {
 #pragma unroll
         for (int i = 0; i < 32; i++) w[i] = x[i] * x[i];
@@ -823,7 +823,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // One lane per block, 64 blocks per workgroup.
 // ------------------------------------------------------------------
 template <int SRC, bool IMAT, int SQ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_iq4_nl(KArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_iq4_nl(KArgs a) {
     constexpr int BYTES = 18;
     __shared__ __attribute__((aligned(16))) uint8_t stage[64 * BYTES];
     __shared__ Iq4Tab iq4tab;
@@ -838,7 +838,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     load_elems<SRC, true, 32>(a.src, row * a.stride + col, x);
     if constexpr (IMAT) {
         const float sigma2 = (2.0f * cascade8_of<32>([&](int i) { return x[i] * x[i]; })) / 32.0f;
-        imatrix_weights<32, true, SQ, 8>(a.qw + col, sigma2, x, a.sqrt, w);
+        imatrix_weights<32, true, SQ>(a.qw + col, sigma2, x, a.sqrt, w);
     } else {
 #pragma unroll
         for (int i = 0; i < 32; i++) w[i] = x[i] * x[i];

@@ -1,5 +1,5 @@
-"""The divisions the kernels build from one reciprocal (qs_device.h: recip,
-quotient): the property their proof needs over every mantissa, and the formats
+"""The divisions and square roots the kernels build from one approximate
+instruction (qs_device.h: recip, quotient, sqrt_root): the property their proof needs over every mantissa, and the formats
 against the oracle where a wave's divisions lie on both sides of the range in
 which they are used."""
 
@@ -27,6 +27,16 @@ def test_reciprocal_and_quotient_over_every_mantissa(qs, dev, e):  # noqa: F811
     # apart, whose quotients are all compared)
     assert 0 < worst < 1 - 2.0**-18
     assert int(out[1]) == 0
+
+
+@pytest.mark.parametrize("k", [-48, -40, -1, 0, 1, 50, 53])
+def test_root_of_every_mantissa(qs, dev, k):  # noqa: F811
+    lib = ctypes.CDLL(str(qs.LIB_PATH.parent / "libqs_calib.so"))
+    lib.qs_calib_sqrt.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    out = torch.zeros(1, dtype=torch.int32, device=dev)
+    assert lib.qs_calib_sqrt(k, out.data_ptr(), None) == 0
+    torch.cuda.synchronize()
+    assert int(out[0]) == 0
 
 
 @pytest.mark.parametrize("imat", [False, True])
