@@ -86,21 +86,24 @@ hipError_t launch_b32(const qs::KArgs& a, hipStream_t st) {
 dim3 sb_grid(const qs::KArgs& a, int lps) { return dim3((unsigned)((a.n_units + 64 / lps - 1) / (64 / lps))); }
 
 // Lanes per group of the make_qkx kernels. A launch of a wave or two per SIMD
-// (256 CUs x 4) takes as long as one wave, whose time is its instruction
-// count: splitting a group over 8 (Q2_K: 4) lanes cuts that to about 0.4 for 2.1
-// times the work, over 4 lanes to 0.5 for 1.5 times. So 8 lanes while that
-// makes at most 2 waves per SIMD (2,048 superblocks), 4 while it makes at most
-// 3 (6,144). Measured, k = 2560, us at 1 / 4 / 8 lanes per group:
-//   Q4_K imatrix  160 superblocks 55.0 / 26.2 / 22.0, 2,040 54.9 / 27.9 / 26.2,
-//                 4,100 57.0 / 40.8 / 45.5, 8,200 60.6 / 59.3 / 72.1
-//   Q4_K          160 29.6 / 14.3 / 12.2, 2,040 29.7 / 15.8 / 15.3,
-//                 4,100 30.4 / 23.3 / 26.1, 8,200 33.1 / 34.2 / 41.0
-//   Q5_K          160 23.7 / 11.8 / 10.6, 2,040 23.8 / 13.1 / 12.8,
-//                 4,100 24.5 / 19.1 / 21.4, 8,200 26.5 / 28.2 / 33.4
-// and Q2_K at 1 / 2 / 4 lanes (2 lanes are never ahead by 5%):
-//   with imatrix  160 38.6 / 29.1 / 24.3, 2,040 40.7 / 31.0 / 29.6, 4,100 41.5 / 43.1 / 47.0
-//   without       160 15.0 / 11.9 / 11.6, 2,040 16.0 / 12.6 / 11.9, 4,100 16.9 / 17.6 / 19.9
-constexpr int64_t kSplit8 = 2048, kSplit4 = 6144;
+// (256 CUs x 4) takes as long as one wave (two waves share a SIMD's issue at
+// full rate), whose time is its instruction count: over 2, 4, 8 lanes a group
+// takes 0.65, 0.5, 0.42 of one wave's time and 1.14, 1.5, 2.1 times the work.
+// So each split is taken up to the 2 or 3 waves per SIMD where the next
+// smaller one overtakes it. Measured, k = 2048 bf16, us at 1 / 2 / 4 / 8 lanes per
+// group for a number of superblocks:
+//   Q4_K imatrix  512 52.8 / 34.3 / 25.7 / 22.7    2,048 53.7 / 36.4 / 26.7 / 26.4
+//                 6,144 54.8 / 42.8 / 41.1 / 53.0  8,192 55.6 / 43.1 / 50.7 / 66.5
+//                 12,288 61.6 / 57.6 / 69.3 / 93.5 16,384 63.0 / 71.4 / 88.0 / 121
+//   Q4_K          2,048 29.4 / 20.7 / 15.3 / 15.4  6,144 30.0 / 24.4 / 23.1 / 29.8
+//                 12,288 34.5 / 32.3 / 38.8 / 52.0 16,384 34.9 / 39.7 / 49.1 / 66.9
+//   Q5_K          2,048 23.6 / 17.0 / 13.1 / 12.9  6,144 24.3 / 20.1 / 19.0 / 24.2
+//                 12,288 28.3 / 26.4 / 31.7 / 42.0 16,384 28.8 / 32.1 / 39.9 / 53.8
+// and Q2_K (16 lanes per superblock at one per group) at 1 / 2 / 4:
+//   with imatrix  512 37.9 / 29.9 / 25.8  2,048 41.1 / 30.8 / 29.0  4,096 40.1 / 34.7 / 42.7
+//                 6,144 45.4 / 43.8 / 56.4  8,192 46.0 / 53.0 / 70.8
+//   without       2,048 15.9 / 12.4 / 12.0  4,096 15.4 / 13.9 / 17.5  6,144 17.2 / 17.9 / 22.9
+constexpr int64_t kSplit8 = 2048, kSplit4 = 6144, kSplit2 = 12288, kSplit2Q2 = 4096;
 
 template <int SRC, bool IMAT, int NMAX, int SQ>
 hipError_t launch_q45(const qs::KArgs& a, hipStream_t st, const qs::Steps& steps) {
@@ -109,6 +112,8 @@ hipError_t launch_q45(const qs::KArgs& a, hipStream_t st, const qs::Steps& steps
         return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 8>, sb_grid(a, 64), wave, st, a, steps, qp_steps(63));
     if (a.n_units <= kSplit4)
         return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 4>, sb_grid(a, 32), wave, st, a, steps, qp_steps(63));
+    if (a.n_units <= kSplit2)
+        return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 2>, sb_grid(a, 16), wave, st, a, steps, qp_steps(63));
     return launch(qs::k_q45_k<SRC, IMAT, NMAX, SQ, 1>, sb_grid(a, 8), wave, st, a, steps, qp_steps(63));
 }
 
@@ -117,6 +122,8 @@ hipError_t launch_q2(const qs::KArgs& a, hipStream_t st, const qs::Steps& steps)
     const dim3 wave(64);
     if (a.n_units <= kSplit8)
         return launch(qs::k_q2_k<SRC, IMAT, SQ, 4>, sb_grid(a, 64), wave, st, a, steps, qp_steps(15));
+    if (a.n_units <= kSplit2Q2)
+        return launch(qs::k_q2_k<SRC, IMAT, SQ, 2>, sb_grid(a, 32), wave, st, a, steps, qp_steps(15));
     return launch(qs::k_q2_k<SRC, IMAT, SQ, 1>, sb_grid(a, 16), wave, st, a, steps, qp_steps(15));
 }
 

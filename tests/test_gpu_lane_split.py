@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 # superblocks per call on both sides of every line of the dispatch, and one
 # superblock, and counts that leave a wave partly empty
-COUNTS = [1, 3, 255, 2048, 2049, 6143, 6144]
+COUNTS = [1, 3, 255, 2048, 2049, 4096, 4097, 6144, 6145, 12288]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -20,7 +20,7 @@ COUNTS = [1, 3, 255, 2048, 2049, 6143, 6144]
 @pytest.mark.parametrize("qtype", ["q2_k", "q4_k", "q5_k"])
 def test_variants_agree_over_the_dispatch(qs, dev, qtype, imat, dtype):  # noqa: F811
     gen = torch.Generator(device="cuda").manual_seed(17)
-    rows = 8200
+    rows = 12300
     x = torch.randn(rows, 256, generator=gen, device=dev) * 0.02
     x *= torch.exp(torch.randn(rows, 1, generator=gen, device=dev))
     x[5] = 0
