@@ -161,6 +161,7 @@ struct HostTab {
 // level (IQ2: level 2) to the grid's level 3 that it makes: it stays valid
 // where such a value's level-3 term is below its level-2 term.
 HostTab build_host_tab(const uint16_t* grid, int gs, int bits, int nwant, int ch, int maxch, int reduce) {
+    const uint16_t pad = bits == 2 ? (uint16_t)gs : 0;     // IQ2: the staged grid's pad point (qs::stage_levels)
     const int nsub = bits == 2 ? 8 : 4, lmask = (1 << bits) - 1, lmax = bits == 2 ? 2 : 7;
     const int ksize = bits == 2 ? 43692 : 4096;
     HostTab t;
@@ -252,12 +253,12 @@ HostTab build_host_tab(const uint16_t* grid, int gs, int bits, int nwant, int ch
                     if (!drop2 && reduce == 2) part.red2.push_back((uint16_t)gj);
                 }
                 const size_t rlen = part.red.size() - rstart, rlen2 = part.red2.size() - rstart2;
-                part.red.resize((part.red.size() + ch - 1) / ch * ch, 0);
-                part.red2.resize((part.red2.size() + ch - 1) / ch * ch, 0);
+                part.red.resize((part.red.size() + ch - 1) / ch * ch, pad);
+                part.red2.resize((part.red2.size() + ch - 1) / ch * ch, pad);
                 t.cinfo_red[c] = (uint32_t)((rstart / ch) << 12) | (uint32_t)rlen;
                 t.cinfo_red2[c] = (uint32_t)((rstart2 / ch) << 12) | (uint32_t)rlen2;
             }
-            part.nbr.resize((part.nbr.size() + ch - 1) / ch * ch, 0);
+            part.nbr.resize((part.nbr.size() + ch - 1) / ch * ch, pad);
             t.cinfo[c] = (uint32_t)((start / ch) << 12) | (uint32_t)len;
             part.ok = part.ok && len < 4096 && len <= (size_t)ch * maxch;
         }

@@ -94,7 +94,9 @@ QS_DEV void static_for(F&& f) {
 }
 
 // Grid levels staged in LDS as bytes 2l+1 (4 per word, NV/4 words per grid
-// point), so a level is one byte-to-float conversion.
+// point), so a level is one byte-to-float conversion. The IQ2 grids (NV = 8) get
+// one more point, GS, which pads their lists' last chunks: levels of 255, a
+// large score in the screen (iq_screen).
 template <int BITS, int NV, int GS, int THREADS = 64>
 QS_DEV void stage_levels(const uint16_t* grid, uint32_t* glv) {
     constexpr int W = NV / 4;
@@ -108,6 +110,7 @@ QS_DEV void stage_levels(const uint16_t* grid, uint32_t* glv) {
         }
         glv[i] = word;
     }
+    if (NV == 8 && threadIdx.x < 2) glv[GS * W + threadIdx.x] = 0xffffffffu;
 }
 
 template <int NV>
@@ -420,6 +423,145 @@ QS_DEV int iq_search(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, uns
     return !want ? 0 : fin ? (int)(r & 0xffffu) : iq_search_miss(ci);     // off-grid: n > 0 iff want
 }
 
+// The two smallest screen scores of one chunk and the grid index of the smaller
+// (GS when no score is below infinity).
+template <int GS>
+QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[IQ2_CH / 2], float sc, const float (&xs)[8],
+                            const float (&ws)[8], float& b1, float& b2, int& g1) {
+    int gi[IQ2_CH];
+    Levels<8> gl[IQ2_CH];
+#pragma unroll
+    for (int j = 0; j < IQ2_CH; j++) {
+        gi[j] = (int)((wd[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+        gl[j] = grid_levels<8>(glds, gi[j]);
+    }
+    b1 = b2 = __builtin_inff();
+    g1 = GS;
+#pragma unroll
+    for (int j = 0; j < IQ2_CH; j++) {
+        float s = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float d = __builtin_fmaf(sc, level<8>(gl[j], e), -xs[e]);
+            s = __builtin_fmaf(ws[e] * d, d, s);
+        }
+        b2 = __builtin_amdgcn_fmed3f(b1, b2, s);
+        g1 = s < b1 ? gi[j] : g1;
+        b1 = fminf(b1, s);
+    }
+}
+
+// iq_search for the IQ2 grids behind a screen. A distance, sum over e of
+// w d^2 with d = sc g - x, takes three instructions a value with fused
+// multiply-adds instead of the five of the reference's roundings, but not the
+// reference's bits. With u = 2^-24, W = sum of w and D an entry's exact distance:
+//   screen:    d and its product carry 3 roundings of a term, the sum 8: 11 u D;
+//   reference: the rounded sc g (at most 7 |sc|) moves d by 7 u |sc|, a term by
+//              14 u w |sc d|, all terms by 14 u |sc| sqrt(W D) <= 7 u (sc^2 W + D);
+//              the other roundings 12 u D: 7 u sc^2 W + 19 u D.
+// So an entry whose score s1 is below every other's by more than
+// 14 u sc^2 W + 60 u s2 (s2 the second smallest) has the strictly smallest
+// reference distance and is the search's result. The screen keeps the two
+// smallest scores of a list and decides where they differ by
+// 64 u (sc^2 W + s2) = 2^-18 (sc^2 W + s2); the other lists (ties, and those with NaN,
+// infinite, overflowing or vanishing sums) go through the exact search, as a
+// wave-wide pass when any lane has one. (Expanding the square to g (A g - B),
+// also three instructions, needs a bound ~100 times larger, and waves ran the
+// exact search too often: IQ2_XXS 1,633 us.) A pad entry scores like a point at
+// levels 255: it can only make a list undecided (as the smallest score its
+// index is not taken).
+// The scores are non-negative, so their bits order them.
+// The chunk arithmetic was about 70% of the searches' instructions. Measured with
+// imatrix: IQ2_XXS bf16 2560x9728 1,177 -> 1,023 us (722 M VALU instructions a
+// launch instead of ~940 M; its 3 waves per SIMD now wait on memory and LDS a
+// third of their cycles), IQ2_S 9728x2560 1,082 -> 1,036, IQ2_XS, with the shorter
+// code check, 1,312 -> 1,030. With OWN against dealing every chunk: IQ2_XXS
+// 1,126 -> 1,088 us on normal weights, IQ2_XS 1,064 -> 1,029; IQ2_S spills 20 more
+// registers and loses a fifth, so it deals every chunk.
+//   sec: LDS, 64 words (the second smallest score of each lane's list)
+template <int OFF, int MAXCH, int GS, bool OWN, bool WL = false, int N>
+QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, unsigned long long* res, uint32_t* sec,
+                     const float (&xv)[N], const float (&wv)[N], float sc, uint32_t ci, bool want, bool& on) {
+    constexpr int NV = 8, CH = IQ2_CH;
+    const int lane = WL ? lane_id() : (int)threadIdx.x;
+    on = (ci & CI_ON_GRID) != 0;
+    const bool listed = want && !on;
+    const int n = listed ? (int)(ci & 0xfffu) : 0;
+    // OWN: a list's first chunk is its own lane's, loaded before the scan and
+    // evaluated without lane exchanges or atomics, and only the others are dealt
+    constexpr int FIRST = OWN ? 1 : 0;
+    uint32_t own[CH / 2] = {};
+    if (OWN && n > 0) iq_load_chunk<CH>(T, (ci >> 12) & 0x7ffffu, own);
+    const int nch = (n + CH - 1) / CH;
+    const int nd = nch > FIRST ? nch - FIRST : 0;
+    const int incl = wave_incl_scan(nd);
+    const int excl = incl - nd;
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    for (int i = 0; i < nd; i++) cmap[excl + i] = (uint8_t)lane;
+    if (OWN && n > 0) {
+        float xs[NV], ws[NV], b1, b2;
+        int g1;
+#pragma unroll
+        for (int e = 0; e < NV; e++) {
+            xs[e] = xv[OFF + e];
+            ws[e] = wv[OFF + e];
+        }
+        iq_chunk_screen<GS>(glds, own, sc, xs, ws, b1, b2, g1);
+        res[lane] = ((unsigned long long)__float_as_uint(b1) << 32) | (unsigned)g1;
+        sec[lane] = __float_as_uint(b2);
+    } else {
+        res[lane] = ~0ull;
+        sec[lane] = 0x7f800000u;
+    }
+    wave_sync<WL>();
+    for (int base = 0; base < total; base += 64) {
+        const int c = base + lane;
+        const bool have = c < total;
+        const int owner = have ? (int)cmap[c] : lane;
+        const int kc = FIRST + c - __shfl(excl, owner);
+        const uint32_t o_ci = (uint32_t)__shfl((int)ci, owner);
+        const float o_sc = __shfl(sc, owner);
+        float xs[NV], ws[NV];
+#pragma unroll
+        for (int e = 0; e < NV; e++) {
+            xs[e] = __shfl(xv[OFF + e], owner);
+            ws[e] = __shfl(wv[OFF + e], owner);
+        }
+        if (have && kc >= FIRST && CH * kc < (int)(o_ci & 0xfffu)) {      // a dealt chunk lies inside its owner's list
+            uint32_t wd[CH / 2];
+            iq_load_chunk<CH>(T, ((o_ci >> 12) & 0x7ffffu) + (size_t)kc, wd);
+            float b1, b2;
+            int g1;
+            iq_chunk_screen<GS>(glds, wd, o_sc, xs, ws, b1, b2, g1);
+            const uint32_t o1 = __float_as_uint(b1);
+            const unsigned long long old =
+                atomicMin(&res[owner], ((unsigned long long)o1 << 32) | (unsigned)g1);
+            // of this chunk's best and the one it met, the larger is not the list's best
+            atomicMin(&sec[owner], min(max((uint32_t)(old >> 32), o1), __float_as_uint(b2)));
+        }
+    }
+    wave_sync<WL>();
+    int gi = (int)(ci & 0xffffu);
+    bool redo = false;
+    if (listed) {
+        const unsigned long long r = res[lane];
+        gi = (int)(r & 0xffffu);
+        const float s1 = __uint_as_float((uint32_t)(r >> 32)), s2 = __uint_as_float(sec[lane]);
+        float W = wv[OFF];
+#pragma unroll
+        for (int e = 1; e < NV; e++) W = W + wv[OFF + e];
+        // a list of one entry has no second (s2 infinite)
+        const float scw = (sc * sc) * W, lim = 0x1p-18f * (scw + (s2 < __builtin_inff() ? s2 : s1));
+        redo = !(s2 - s1 > lim && lim >= 0x1p-100f && lim <= 0x1p100f && fabsf(sc) <= 0x1p30f && gi < GS);
+    }
+    if (wave_any(redo)) {
+        bool dummy;
+        const int r = iq_search<2, NV, OFF, CH, MAXCH, WL>(T, glds, cmap, res, xv, wv, sc, ci, redo, dummy);
+        gi = redo ? r : gi;
+    }
+    return on || want ? gi : 0;
+}
+
 // Every subgroup whose search found no finite distance (rare: an infinite
 // or NaN weight, value or scale) gets torch's argmin from an in-order scan
 // of its list; the wave skips this when none did. OUTLINE calls the scan
@@ -599,10 +741,11 @@ template <int SRC, int SQ>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_iq2_xxs(KArgs a, IqTabDev T, QpSteps qp4, IqSteps sweep) {
     constexpr int LPS = 8, SPW = 8, BYTES = 66;
     __shared__ IqLds<SPW, BYTES> s;
-    __shared__ __align__(16) uint32_t glds[256 * 2];
+    __shared__ __align__(16) uint32_t glds[256 * 2 + 2];
     __shared__ uint8_t cmap[64 * IQ2_256_MAXCH];
     __shared__ unsigned long long res[64];
     stage_levels<2, 8, 256>(T.grid, glds);
+    uint32_t* sec = reinterpret_cast<uint32_t*>(s.v);     // free between the weights and the packing
     const SbPos p = sb_pos<LPS, 32>(a.n_units, a.units_per_row, a.stride);
     const int slot = p.slot, g = p.g;
     float x[32], w[32], waux[32], xval[32];
@@ -632,7 +775,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         uint32_t ci[4];
         iq_codes<2, 8, 4, 2>(T, xval, inv, ci, sc);
         static_for<0, 4>([&](auto S) {
-            gi[S] = iq_search<2, 8, 8 * S, IQ2_CH, IQ2_256_MAXCH>(T, glds, cmap, res, xval, waux, sc, ci[S], true, on);
+            gi[S] = iq_screen<8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on);
         });
         iq_rescan<8, IQ2_CH, true>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
@@ -653,7 +796,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         uint32_t ci[4];
         iq_codes<2, 8, 4, 2>(T, xval, inv, ci, scale);
         static_for<0, 4>([&](auto S) {
-            gp[S] = iq_search<2, 8, 8 * S, IQ2_CH, IQ2_256_MAXCH>(T, glds, cmap, res, xval, waux, scale, ci[S], proj, on);
+            gp[S] = iq_screen<8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S], proj, on);
         });
         iq_rescan<8, IQ2_CH, true>(T, glds, xval, waux, scale, gp);
         float sumqx, sumq2;
@@ -714,7 +857,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
     constexpr int LPS = 16, SPW = 4, BYTES = IS_S ? 82 : 74, GS = IS_S ? 1024 : 512;
     constexpr int MAXCH = IS_S ? IQ2_1024_MAXCH : IQ2_512_MAXCH;
     __shared__ IqLds<SPW, BYTES> s_w[WPG];
-    __shared__ __align__(16) uint32_t glds[GS * 2];
+    __shared__ __align__(16) uint32_t glds[GS * 2 + 2];
     __shared__ int wlds_w[WPG][SPW][16][2];
     __shared__ uint8_t cmap_w[WPG][64 * MAXCH];
     __shared__ unsigned long long res_w[WPG][64];
@@ -726,6 +869,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
     constexpr bool WL = WPG > 1;
     stage_levels<2, 8, GS, 64 * WPG>(T.grid, glds);
     if constexpr (WL) __syncthreads();            // the grid is every wave's
+    uint32_t* sec = reinterpret_cast<uint32_t*>(s.v);     // free between the weights and the packing
     const SbPos p = sb_pos<LPS, 16, WPG>(a.n_units, a.units_per_row, a.stride);
     const int slot = p.slot, g = p.g;
     float x[16], w[16], waux[16], xval[16];
@@ -755,8 +899,8 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         bool on[2];
         uint32_t ci[2];
         iq_codes<2, 8, 2, IS_S ? 0 : 1>(T, xval, inv, ci, sc);
-        gi[0] = iq_search<2, 8, 0, IQ2_CH, MAXCH, WL>(T, glds, cmap, res, xval, waux, sc, ci[0], true, on[0]);
-        gi[1] = iq_search<2, 8, 8, IQ2_CH, MAXCH, WL>(T, glds, cmap, res, xval, waux, sc, ci[1], true, on[1]);
+        gi[0] = iq_screen<0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[0], true, on[0]);
+        gi[1] = iq_screen<8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[1], true, on[1]);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
         iq_tree_sums<2, 8, 2>(glds, gi, w, xval, sumqx, sumq2);
@@ -779,9 +923,9 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         uint32_t ci[2];
         iq_codes<2, 8, 2, IS_S ? 0 : 1>(T, xval, inv, ci, scale);
         int r[2];
-        r[0] = iq_search<2, 8, 0, IQ2_CH, MAXCH, WL>(T, glds, cmap, res, xval, waux, scale, ci[0],
+        r[0] = iq_screen<0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[0],
                                                      need && !og[0], on);
-        r[1] = iq_search<2, 8, 8, IQ2_CH, MAXCH, WL>(T, glds, cmap, res, xval, waux, scale, ci[1],
+        r[1] = iq_screen<8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[1],
                                                      need && !og[1], on);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, scale, r);
         if (need && !og[0]) win[0] = r[0];
