@@ -161,7 +161,7 @@ struct HostTab {
 // level (IQ2: level 2) to the grid's level 3 that it makes: it stays valid
 // where such a value's level-3 term is below its level-2 term.
 HostTab build_host_tab(const uint16_t* grid, int gs, int bits, int nwant, int ch, int maxch, int reduce) {
-    const uint16_t pad = bits == 2 ? (uint16_t)gs : 0;     // IQ2: the staged grid's pad point (qs::stage_levels)
+    const uint16_t pad = (uint16_t)gs;                     // the staged grid's pad point (qs::stage_levels)
     const int nsub = bits == 2 ? 8 : 4, lmask = (1 << bits) - 1, lmax = bits == 2 ? 2 : 7;
     const int ksize = bits == 2 ? 43692 : 4096;
     HostTab t;

@@ -94,9 +94,9 @@ QS_DEV void static_for(F&& f) {
 }
 
 // Grid levels staged in LDS as bytes 2l+1 (4 per word, NV/4 words per grid
-// point), so a level is one byte-to-float conversion. The IQ2 grids (NV = 8) get
-// one more point, GS, which pads their lists' last chunks: levels of 255, a
-// large score in the screen (iq_screen).
+// point), so a level is one byte-to-float conversion. One more point, GS, pads
+// the lists' last chunks: levels of 255, a large score in the screen
+// (iq_screen).
 template <int BITS, int NV, int GS, int THREADS = 64>
 QS_DEV void stage_levels(const uint16_t* grid, uint32_t* glv) {
     constexpr int W = NV / 4;
@@ -110,7 +110,7 @@ QS_DEV void stage_levels(const uint16_t* grid, uint32_t* glv) {
         }
         glv[i] = word;
     }
-    if (NV == 8 && threadIdx.x < 2) glv[GS * W + threadIdx.x] = 0xffffffffu;
+    if (threadIdx.x < W) glv[GS * W + threadIdx.x] = 0xffffffffu;
 }
 
 template <int NV>
@@ -425,24 +425,24 @@ QS_DEV int iq_search(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, uns
 
 // The two smallest screen scores of one chunk and the grid index of the smaller
 // (GS when no score is below infinity).
-template <int GS>
-QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[IQ2_CH / 2], float sc, const float (&xs)[8],
-                            const float (&ws)[8], float& b1, float& b2, int& g1) {
-    int gi[IQ2_CH];
-    Levels<8> gl[IQ2_CH];
+template <int NV, int CH, int GS>
+QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[CH / 2], float sc, const float (&xs)[NV],
+                            const float (&ws)[NV], float& b1, float& b2, int& g1) {
+    int gi[CH];
+    Levels<NV> gl[CH];
 #pragma unroll
-    for (int j = 0; j < IQ2_CH; j++) {
+    for (int j = 0; j < CH; j++) {
         gi[j] = (int)((wd[j >> 1] >> (16 * (j & 1))) & 0xffffu);
-        gl[j] = grid_levels<8>(glds, gi[j]);
+        gl[j] = grid_levels<NV>(glds, gi[j]);
     }
     b1 = b2 = __builtin_inff();
     g1 = GS;
 #pragma unroll
-    for (int j = 0; j < IQ2_CH; j++) {
+    for (int j = 0; j < CH; j++) {
         float s = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const float d = __builtin_fmaf(sc, level<8>(gl[j], e), -xs[e]);
+        for (int e = 0; e < NV; e++) {
+            const float d = __builtin_fmaf(sc, level<NV>(gl[j], e), -xs[e]);
             s = __builtin_fmaf(ws[e] * d, d, s);
         }
         b2 = __builtin_amdgcn_fmed3f(b1, b2, s);
@@ -451,16 +451,18 @@ QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[IQ2_CH / 
     }
 }
 
-// iq_search for the IQ2 grids behind a screen. A distance, sum over e of
+// iq_search behind a screen. A distance, sum over e of
 // w d^2 with d = sc g - x, takes three instructions a value with fused
 // multiply-adds instead of the five of the reference's roundings, but not the
 // reference's bits. With u = 2^-24, W = sum of w and D an entry's exact distance:
-//   screen:    d and its product carry 3 roundings of a term, the sum 8: 11 u D;
+//   screen:    d and its product carry 3 roundings of a term, the sum 8: 11 u D
+//              (IQ3: 4 values, 7 u D);
 //   reference: the rounded sc g (at most 7 |sc|) moves d by 7 u |sc|, a term by
 //              14 u w |sc d|, all terms by 14 u |sc| sqrt(W D) <= 7 u (sc^2 W + D);
-//              the other roundings 12 u D: 7 u sc^2 W + 19 u D.
+//              the other roundings 12 u D: 7 u sc^2 W + 19 u D (IQ3: levels to
+//              15, 15 u sc^2 W + 23 u D).
 // So an entry whose score s1 is below every other's by more than
-// 14 u sc^2 W + 60 u s2 (s2 the second smallest) has the strictly smallest
+// 30 u sc^2 W + 60 u s2 (s2 the second smallest) has the strictly smallest
 // reference distance and is the search's result. The screen keeps the two
 // smallest scores of a list and decides where they differ by
 // 64 u (sc^2 W + s2) = 2^-18 (sc^2 W + s2); the other lists (ties, and those with NaN,
@@ -475,14 +477,15 @@ QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[IQ2_CH / 
 // imatrix: IQ2_XXS bf16 2560x9728 1,177 -> 1,023 us (722 M VALU instructions a
 // launch instead of ~940 M; its 3 waves per SIMD now wait on memory and LDS a
 // third of their cycles), IQ2_S 9728x2560 1,082 -> 1,036, IQ2_XS, with the shorter
-// code check, 1,312 -> 1,030. With OWN against dealing every chunk: IQ2_XXS
+// code check, 1,312 -> 1,030; IQ3_XXS 9728x2560 1,449 -> 1,317, 1024x2560 192 -> 177,
+// IQ3_S 9728x2560 962 -> 947. With OWN against dealing every chunk: IQ2_XXS
 // 1,126 -> 1,088 us on normal weights, IQ2_XS 1,064 -> 1,029; IQ2_S spills 20 more
 // registers and loses a fifth, so it deals every chunk.
 //   sec: LDS, 64 words (the second smallest score of each lane's list)
-template <int OFF, int MAXCH, int GS, bool OWN, bool WL = false, int N>
+template <int BITS, int OFF, int MAXCH, int GS, bool OWN, bool WL = false, int N>
 QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, unsigned long long* res, uint32_t* sec,
                      const float (&xv)[N], const float (&wv)[N], float sc, uint32_t ci, bool want, bool& on) {
-    constexpr int NV = 8, CH = IQ2_CH;
+    constexpr int NV = BITS == 2 ? 8 : 4, CH = BITS == 2 ? IQ2_CH : IQ3_CH;
     const int lane = WL ? lane_id() : (int)threadIdx.x;
     on = (ci & CI_ON_GRID) != 0;
     const bool listed = want && !on;
@@ -506,7 +509,7 @@ QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, uns
             xs[e] = xv[OFF + e];
             ws[e] = wv[OFF + e];
         }
-        iq_chunk_screen<GS>(glds, own, sc, xs, ws, b1, b2, g1);
+        iq_chunk_screen<NV, CH, GS>(glds, own, sc, xs, ws, b1, b2, g1);
         res[lane] = ((unsigned long long)__float_as_uint(b1) << 32) | (unsigned)g1;
         sec[lane] = __float_as_uint(b2);
     } else {
@@ -532,7 +535,7 @@ QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, uns
             iq_load_chunk<CH>(T, ((o_ci >> 12) & 0x7ffffu) + (size_t)kc, wd);
             float b1, b2;
             int g1;
-            iq_chunk_screen<GS>(glds, wd, o_sc, xs, ws, b1, b2, g1);
+            iq_chunk_screen<NV, CH, GS>(glds, wd, o_sc, xs, ws, b1, b2, g1);
             const uint32_t o1 = __float_as_uint(b1);
             const unsigned long long old =
                 atomicMin(&res[owner], ((unsigned long long)o1 << 32) | (unsigned)g1);
@@ -556,7 +559,7 @@ QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, uns
     }
     if (wave_any(redo)) {
         bool dummy;
-        const int r = iq_search<2, NV, OFF, CH, MAXCH, WL>(T, glds, cmap, res, xv, wv, sc, ci, redo, dummy);
+        const int r = iq_search<BITS, NV, OFF, CH, MAXCH, WL>(T, glds, cmap, res, xv, wv, sc, ci, redo, dummy);
         gi = redo ? r : gi;
     }
     return on || want ? gi : 0;
@@ -775,7 +778,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         uint32_t ci[4];
         iq_codes<2, 8, 4, 2>(T, xval, inv, ci, sc);
         static_for<0, 4>([&](auto S) {
-            gi[S] = iq_screen<8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on);
+            gi[S] = iq_screen<2, 8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on);
         });
         iq_rescan<8, IQ2_CH, true>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
@@ -796,7 +799,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         uint32_t ci[4];
         iq_codes<2, 8, 4, 2>(T, xval, inv, ci, scale);
         static_for<0, 4>([&](auto S) {
-            gp[S] = iq_screen<8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S], proj, on);
+            gp[S] = iq_screen<2, 8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S], proj, on);
         });
         iq_rescan<8, IQ2_CH, true>(T, glds, xval, waux, scale, gp);
         float sumqx, sumq2;
@@ -899,8 +902,8 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         bool on[2];
         uint32_t ci[2];
         iq_codes<2, 8, 2, IS_S ? 0 : 1>(T, xval, inv, ci, sc);
-        gi[0] = iq_screen<0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[0], true, on[0]);
-        gi[1] = iq_screen<8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[1], true, on[1]);
+        gi[0] = iq_screen<2, 0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[0], true, on[0]);
+        gi[1] = iq_screen<2, 8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[1], true, on[1]);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
         iq_tree_sums<2, 8, 2>(glds, gi, w, xval, sumqx, sumq2);
@@ -923,9 +926,9 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         uint32_t ci[2];
         iq_codes<2, 8, 2, IS_S ? 0 : 1>(T, xval, inv, ci, scale);
         int r[2];
-        r[0] = iq_screen<0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[0],
+        r[0] = iq_screen<2, 0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[0],
                                                      need && !og[0], on);
-        r[1] = iq_screen<8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[1],
+        r[1] = iq_screen<2, 8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[1],
                                                      need && !og[1], on);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, scale, r);
         if (need && !og[0]) win[0] = r[0];
@@ -1015,12 +1018,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
     constexpr int LPS = 8 * LPG, SPW = 64 / LPS, BYTES = IS_S ? 110 : 98, GS = IS_S ? 512 : 256;
     constexpr int SMASK = IS_S ? 255 : 127;
     __shared__ IqLds<SPW, BYTES> s;
-    __shared__ __align__(16) uint32_t glds[GS];
+    __shared__ __align__(16) uint32_t glds[GS + 1];
     __shared__ int act_lds[SPW][8];
     constexpr int MAXCH = IS_S ? IQ3_512_MAXCH : IQ3_256_MAXCH;
     __shared__ uint8_t cmap[64 * MAXCH];
     __shared__ unsigned long long res[64];
     stage_levels<3, 4, GS>(T.grid, glds);
+    uint32_t* sec = reinterpret_cast<uint32_t*>(s.v);     // free between the weights and the packing
     const SbPos p = sb_pos<LPS, VPL>(a.n_units, a.units_per_row, a.stride);
     const int slot = p.slot, grp = p.g / LPG, q = p.g % LPG;
     float x[VPL], w[VPL], waux[VPL], xval[VPL];
@@ -1068,7 +1072,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
         uint32_t ci[NSL];
         iq_codes<3, 4, NSL, 1>(T, xval, inv, ci, sc);
         static_for<0, NSL>([&](auto S) {
-            gi[S] = iq_search<3, 4, 4 * S, IQ3_CH, MAXCH>(T, glds, cmap, res, xval, waux, sc, ci[S], true, on[S]);
+            gi[S] = iq_screen<3, 4 * S, MAXCH, GS, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on[S]);
         });
         iq_rescan<4, IQ3_CH, true>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
@@ -1097,7 +1101,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
         uint32_t ci[NSL];
         iq_codes<3, 4, NSL, 1>(T, xval, inv2, ci, scale);
         static_for<0, NSL>([&](auto S) {
-            w2[S] = iq_search<3, 4, 4 * S, IQ3_CH, MAXCH>(T, glds, cmap, res, xval, waux, scale, ci[S],
+            w2[S] = iq_screen<3, 4 * S, MAXCH, GS, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S],
                                                           redo && (IS_S || !og[S]), on[S]);
         });
         iq_rescan<4, IQ3_CH, true>(T, glds, xval, waux, scale, w2);
