@@ -438,6 +438,10 @@ QS_DEV QxResult qx_fit(const float (&x)[N], const float (&w)[N], int nmax, const
     return r;
 }
 
+// floats of LDS a 19-trial make_qx (qx_fit_spread, NS = 18) and a 16-trial IQ4
+// search exchange per group, odd so that groups start in different banks
+constexpr int QX_XCH = 3 * 19, IQ4_XCH = 33;
+
 // make_qx_quants_eager for one superblock's N sub-block scales, spread over
 // P consecutive lanes (c = 0..P-1) that all hold x and w, for NS candidates
 // (the host's steps.n). A trial's levels and sums depend only on its iscale,
@@ -621,8 +625,12 @@ QS_DEV void iq4_pack(const float (&x)[32], float id, const Iq4Tab& t, uint32_t (
 // imatrix weights taken 8 at a time gives the imatrix kernels a fourth wave
 // per SIMD (6-7% faster); the kernels without imatrix were 4% slower at 4
 // waves and stage all 32 (CH = 32, 3 waves).
-template <int CH>
-QS_DEV float iq4_scale_search(const float (&x)[32], const float (&w)[32], const Iq4Tab& tab) {
+// LPG > 1: the LPG lanes c = 0 .. LPG - 1 of a block all hold it, lane c forms the
+// sums of trials c, c + LPG, ... (a trial does not depend on earlier accepts),
+// they meet in xch (32 floats of LDS), and every lane runs the accept chain in
+// trial order.
+template <int CH, int LPG>
+QS_DEV float iq4_scale_search(const float (&x)[32], const float (&w)[32], const Iq4Tab& tab, int c0, float* xch) {
     float amax;
     const float mx = absmax_first(x, amax);
     const bool live = fabsf(mx) >= GROUP_MAX_EPS;
@@ -649,13 +657,29 @@ QS_DEV float iq4_scale_search(const float (&x)[32], const float (&w)[32], const 
         }
     };
     float sumqx, sumq2;
-    sums(id0, sumqx, sumq2);
+    if constexpr (LPG > 1) {
+#pragma unroll 1
+        for (int e = c0; e < 16; e += LPG) {
+            sums(e == 0 ? id0 : rdiv((float)(e - 8 - 127), mxs), sumqx, sumq2);
+            xch[2 * e] = sumqx;
+            xch[2 * e + 1] = sumq2;
+        }
+        wave_sync();
+        sumqx = xch[0];
+        sumq2 = xch[1];
+    } else {
+        sums(id0, sumqx, sumq2);
+    }
     float d = sumq2 > 0 ? sumqx / sumq2 : 0.0f;
     float best = d * sumqx;
 #pragma unroll 1
     for (int itry = -7; itry <= 7; itry++) {
-        const float idv = rdiv((float)(itry - 127), mxs);
-        sums(idv, sumqx, sumq2);
+        if constexpr (LPG > 1) {
+            sumqx = xch[2 * (itry + 8)];
+            sumq2 = xch[2 * (itry + 8) + 1];
+        } else {
+            sums(rdiv((float)(itry - 127), mxs), sumqx, sumq2);
+        }
         if (sumq2 > 0 && sumqx * sumqx > best * sumq2) {
             const float nd = sumqx / sumq2;
             d = nd;

@@ -324,9 +324,10 @@ QS_DEV float group_cascade8(const float (&v)[V], float* stage, int gl) {
 // wave's superblocks at a time (half the LDS). Every lane takes part in both
 // rounds, the wave barriers included; lanes of the other half compute the
 // same sums from the same staged values and discard them.
-template <int LPS, int SPW, int GROUP, bool WL = false>
+// With LPG > 1 the LPG lanes of a group hold the same GROUP values.
+template <int LPS, int SPW, int GROUP, bool WL = false, int LPG = 1>
 QS_DEV float sb_sumsq_halves(float (*v)[QK_K], float (*tmp)[40], const float (&x)[GROUP], int slot, int g) {
-    static_assert(GROUP * LPS == QK_K, "the lanes of a superblock cover its values");
+    static_assert(GROUP * LPS == QK_K * LPG, "the lanes of a superblock cover its values");
     constexpr int H = SPW / 2;
     const int hs = slot % H;
     float sum = 0.0f;
@@ -335,7 +336,7 @@ QS_DEV float sb_sumsq_halves(float (*v)[QK_K], float (*tmp)[40], const float (&x
         const bool mine = slot / H == r;
         if (mine) {
 #pragma unroll
-            for (int i = 0; i < GROUP; i++) v[hs][GROUP * g + i] = x[i] * x[i];
+            for (int i = 0; i < GROUP; i++) v[hs][GROUP * (g / LPG) + i] = x[i] * x[i];
         }
         wave_sync<WL>();
         const float t = sb_cascade8_256<LPS, WL>(v[hs], tmp[hs], g);
@@ -553,12 +554,17 @@ __global__ __launch_bounds__(64) void k_q6_k(KArgs a, Steps steps) {
 // ------------------------------------------------------------------
 // Q3_K  (q3_k.py:23-78)
 // ------------------------------------------------------------------
-template <int SRC, bool IMAT, int SQ>
+template <int SRC, bool IMAT, int SQ, int LPG>
+// LPG lanes per group: every one holds the group's 16 values, and make_qx's
+// trials, which do not depend on each other, are spread over them (with an
+// imatrix only: make_q3's passes are one chain)
 __global__ __launch_bounds__(64) void k_q3_k(KArgs a, Steps steps4, Steps steps32) {
-    constexpr int LPS = 16, SPW = 4, BYTES = 110;
+    static_assert(IMAT || LPG == 1, "make_q3 has no trials to spread");
+    constexpr int LPS = 16 * LPG, SPW = 64 / LPS, BYTES = 110;
     __shared__ SbLds<SPW, BYTES> s;
-    const SbPos p = sb_pos<LPS, 16>(a.n_units, a.units_per_row, a.stride);
-    const int slot = p.slot, g = p.g;
+    __shared__ float xch[LPG > 1 ? SPW * 16 * QX_XCH : 1];
+    const SbPos p = sb_pos<LPS, 16, 1, LPG>(a.n_units, a.units_per_row, a.stride);
+    const int slot = p.slot, gl = p.g, g = gl / LPG;       // superblock, lane in it, its group
     float x[16];
     load_elems<SRC, true, 16>(a.src, p.elem, x);
 
@@ -588,7 +594,9 @@ __global__ __launch_bounds__(64) void k_q3_k(KArgs a, Steps steps4, Steps steps3
         wave_sync();
         const float sigma2 = (2.0f * sb_seq_256(s.v[slot])) / 256.0f;
         imatrix_weights<16, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
-        const QxResult r = qx_fit<16>(x, w, 4, steps4);
+        QxResult r;
+        if constexpr (LPG == 1) r = qx_fit<16>(x, w, 4, steps4);
+        else r = qx_fit_spread<16, LPG, 18>(x, w, 4, steps4, gl % LPG, xch + QX_XCH * (16 * slot + g));
 #pragma unroll
         for (int i = 0; i < 16; i++) Lg[i] = qx_level(r, x[i], 4.0f);
         s.sc[slot][g] = r.scale;
@@ -596,15 +604,15 @@ __global__ __launch_bounds__(64) void k_q3_k(KArgs a, Steps steps4, Steps steps3
         wave_sync();
         {
             // make_qx over the 16 sub-block scales, its 19 trials spread over
-            // the superblock's 16 lanes; the exchange reuses the x^2 staging
+            // the superblock's lanes; the exchange reuses the x^2 staging
             float sc16[16], sw16[16];
 #pragma unroll
             for (int j = 0; j < 16; j++) {
                 sc16[j] = s.sc[slot][j];
                 sw16[j] = s.sw[slot][j];
             }
-            const QxResult r2 = qx_fit_spread<16, 16, 18>(sc16, sw16, 32, steps32, g, s.v[slot]);
-            if (g == 0) s.hdr[slot][0] = r2.scale;
+            const QxResult r2 = qx_fit_spread<16, LPS, 18>(sc16, sw16, 32, steps32, gl, s.v[slot]);
+            if (gl == 0) s.hdr[slot][0] = r2.scale;
             s.ls[slot][g] = (int)qx_level(r2, s.sc[slot][g], 32.0f);
         }
         wave_sync();
@@ -627,24 +635,22 @@ __global__ __launch_bounds__(64) void k_q3_k(KArgs a, Steps steps4, Steps steps3
     const uint32_t* L = reinterpret_cast<const uint32_t*>(s.L[slot]);
     const int* LS = s.ls[slot];
     uint8_t* o = s.out + slot * BYTES;
-    {
-        uint32_t v = 0;                                   // hmask bytes 2 g, 2 g + 1: bit 2 of the levels
+    if (LPG == 1 || gl < 16) {
+        uint32_t v = 0;                                   // hmask bytes 2 gl, 2 gl + 1: bit 2 of the levels
 #pragma unroll
         for (int b = 0; b < 8; b++)
-            v |= (((uint32_t)reinterpret_cast<const uint16_t*>(L)[16 * b + g] >> 2) & 0x0101u) << b;
-        *reinterpret_cast<uint16_t*>(o + 2 * g) = (uint16_t)v;
-    }
-    {
-        const uint32_t* q = L + 32 * (g >> 3) + (g & 7);  // qs bytes 4 g .. + 3: bits 0-1
-        uint32_t v = 0;
+            v |= (((uint32_t)reinterpret_cast<const uint16_t*>(L)[16 * b + gl] >> 2) & 0x0101u) << b;
+        *reinterpret_cast<uint16_t*>(o + 2 * gl) = (uint16_t)v;
+        const uint32_t* q = L + 32 * (gl >> 3) + (gl & 7);  // qs bytes 4 gl .. + 3: bits 0-1
+        v = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) v |= (q[8 * i] & 0x03030303u) << (2 * i);
-        store_u16x2(o + 32 + 4 * g, v);
+        store_u16x2(o + 32 + 4 * gl, v);
     }
-    if (g < 8) o[96 + g] = (uint8_t)((LS[g] & 15) | ((LS[g + 8] & 15) << 4));
-    if (g < 4)
-        o[104 + g] = (uint8_t)((LS[g] >> 4) | ((LS[4 + g] >> 4) << 2) | ((LS[8 + g] >> 4) << 4) | ((LS[12 + g] >> 4) << 6));
-    if (g == 0) *reinterpret_cast<uint16_t*>(o + 108) = (uint16_t)f16_bits(d16);
+    if (gl < 8) o[96 + gl] = (uint8_t)((LS[gl] & 15) | ((LS[gl + 8] & 15) << 4));
+    if (gl < 4)
+        o[104 + gl] = (uint8_t)((LS[gl] >> 4) | ((LS[4 + gl] >> 4) << 2) | ((LS[8 + gl] >> 4) << 4) | ((LS[12 + gl] >> 4) << 6));
+    if (gl == 0) *reinterpret_cast<uint16_t*>(o + 108) = (uint16_t)f16_bits(d16);
     wave_sync();
     sb_store(s, a);
 }
@@ -757,27 +763,29 @@ __global__ __launch_bounds__(64) void k_q2_k(KArgs a, Steps steps, QpSteps qps) 
 // ------------------------------------------------------------------
 // IQ4_XS  (iq4_xs.py:149-188)
 // ------------------------------------------------------------------
-template <int SRC, bool IMAT, int SQ>
+template <int SRC, bool IMAT, int SQ, int LPG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_iq4_xs(KArgs a) {
-    constexpr int LPS = 8, SPW = 8, BYTES = 136;
+    constexpr int LPS = 8 * LPG, SPW = 64 / LPS, BYTES = 136;
     // LDS is what limits this kernel's residency: the imatrix path stages x^2
     // for sigma2 half the wave's superblocks at a time, the other stages none
     __shared__ SbLds<SPW, BYTES, IMAT ? SPW / 2 : 1> s;
     __shared__ Iq4Tab iq4tab;
+    __shared__ float xch[LPG > 1 ? SPW * 8 * IQ4_XCH : 1];
     iq4_load_tab(iq4tab);
-    const SbPos p = sb_pos<LPS, 32>(a.n_units, a.units_per_row, a.stride);
-    const int slot = p.slot, g = p.g;
+    // LPG lanes per block share its trials; every one holds its 32 values
+    const SbPos p = sb_pos<LPS, 32, 1, LPG>(a.n_units, a.units_per_row, a.stride);
+    const int slot = p.slot, gl = p.g, g = gl / LPG;
     float x[32], w[32];
     load_elems<SRC, true, 32>(a.src, p.elem, x);
     if constexpr (IMAT) {
-        const float sigma2 = (2.0f * sb_sumsq_halves<LPS, SPW, 32>(s.v, s.tmp, x, slot, g)) / 256.0f;
+        const float sigma2 = (2.0f * sb_sumsq_halves<LPS, SPW, 32, false, LPG>(s.v, s.tmp, x, slot, gl)) / 256.0f;
         imatrix_weights<32, true, SQ>(a.qw + p.col, sigma2, x, a.sqrt, w);
     } else {
 #pragma unroll
         for (int i = 0; i < 32; i++) w[i] = x[i] * x[i];
     }
     if constexpr (!IMAT) wave_sync();          // iq4tab ready (the imatrix path synced above)
-    const float scale = iq4_scale_search<IMAT ? 16 : 32>(x, w, iq4tab);
+    const float scale = iq4_scale_search<IMAT ? 16 : 32, LPG>(x, w, iq4tab, gl % LPG, xch + IQ4_XCH * (8 * slot + g));
     s.sc[slot][g] = scale;
     wave_sync();
     float sc8[8];
@@ -802,8 +810,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     oq[0] = q[0] | ((uint64_t)q[1] << 32);
     oq[1] = q[2] | ((uint64_t)q[3] << 32);
     const int* LS = s.ls[slot];
-    if (g < 4) o[4 + g] = (uint8_t)((LS[2 * g] & 15) | ((LS[2 * g + 1] & 15) << 4));
-    if (g == 0) {
+    if (gl < 4) o[4 + gl] = (uint8_t)((LS[2 * gl] & 15) | ((LS[2 * gl + 1] & 15) << 4));
+    if (gl == 0) {
         uint32_t h = 0;
 #pragma unroll
         for (int b = 0; b < 8; b++) h |= (uint32_t)(LS[b] >> 4) << (2 * b);
@@ -844,7 +852,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         for (int i = 0; i < 32; i++) w[i] = x[i] * x[i];
     }
     wave_sync();                                 // iq4tab ready
-    const float scale = iq4_scale_search<IMAT ? 16 : 32>(x, w, iq4tab);
+    const float scale = iq4_scale_search<IMAT ? 16 : 32, 1>(x, w, iq4tab, 0, nullptr);
     const float id = scale != 0.0f ? 1.0f / scale : 0.0f;
     uint8_t* o = stage + lane * BYTES;
     const uint32_t h = f16_bits(scale);

@@ -127,6 +127,23 @@ hipError_t launch_q2(const qs::KArgs& a, hipStream_t st, const qs::Steps& steps)
     return launch(qs::k_q2_k<SRC, IMAT, SQ, 1>, sb_grid(a, 16), wave, st, a, steps, qp_steps(15));
 }
 
+// Four lanes per group for the trials of Q3_K with an imatrix and IQ4_XS, where the
+// launch has few waves (the reason is that of launch_q45; each lane repeats the
+// weights and the levels, so the work grows faster). Measured, k = 2048 bf16, us at
+// 1 / 4 lanes per group:
+//   Q3_K imatrix    512 superblocks 14.9 / 12.6  2,048 16.0 / 13.8  3,072 15.6 / 16.6
+//   IQ4_XS imatrix  512 18.5 / 12.0  4,096 20.2 / 14.3  6,144 20.3 / 17.4  10,240 23.4 / 25.2
+//   IQ4_XS          512 15.3 / 11.0  4,096 16.7 / 11.1  6,144 16.4 / 12.3  12,288 18.2 / 18.2
+// (Q6_K gained 8% at most, 12.1 / 11.1 at 2,048, and is not split.)
+constexpr int64_t kSpreadQ3 = 2048, kSpreadIq4 = 6144;
+
+template <int SRC, bool IMAT, int SQ>
+hipError_t launch_iq4(const qs::KArgs& a, hipStream_t st) {
+    const dim3 wave(64);
+    if (a.n_units <= kSpreadIq4) return launch(qs::k_iq4_xs<SRC, IMAT, SQ, 4>, sb_grid(a, 32), wave, st, a);
+    return launch(qs::k_iq4_xs<SRC, IMAT, SQ, 1>, sb_grid(a, 8), wave, st, a);
+}
+
 // SQ: the host whose square-root rounding the weights take (qs::SQ_*);
 // kernels whose weights take no square root are instantiated once (SQ_IEEE).
 template <int SRC, int SQ>
@@ -156,14 +173,15 @@ hipError_t launch_type(int type, bool imat, const qs::KArgs& a, hipStream_t st,
         return imat ? launch(k_q6_k<SRC, true>, sb4, wave, st, a, qx_steps(32))
                     : launch(k_q6_k<SRC, false>, sb4, wave, st, a, qx_steps(32));
     case QS_TYPE_Q3_K:
-        return imat ? launch(k_q3_k<SRC, true, SQ>, sb4, wave, st, a, qx_steps(4), qx_steps(32))
-                    : launch(k_q3_k<SRC, false, SQ_IEEE>, sb4, wave, st, a, qx_steps(4), qx_steps(32));
+        if (!imat) return launch(k_q3_k<SRC, false, SQ_IEEE, 1>, sb4, wave, st, a, qx_steps(4), qx_steps(32));
+        if (a.n_units <= kSpreadQ3)
+            return launch(k_q3_k<SRC, true, SQ, 4>, sb_grid(a, 64), wave, st, a, qx_steps(4), qx_steps(32));
+        return launch(k_q3_k<SRC, true, SQ, 1>, sb4, wave, st, a, qx_steps(4), qx_steps(32));
     case QS_TYPE_Q2_K:
         return imat ? launch_q2<SRC, true, SQ>(a, st, qkx_steps(-0.9f, 0.05f, 36, 3))
                     : launch_q2<SRC, false, SQ_IEEE>(a, st, qkx_steps(-0.5f, 0.1f, 15, 3));
     case QS_TYPE_IQ4_XS:
-        return imat ? launch(k_iq4_xs<SRC, true, SQ>, sb8, wave, st, a)
-                    : launch(k_iq4_xs<SRC, false, SQ_IEEE>, sb8, wave, st, a);
+        return imat ? launch_iq4<SRC, true, SQ>(a, st) : launch_iq4<SRC, false, SQ_IEEE>(a, st);
     case QS_TYPE_IQ2_XXS: {
         // candidate numerators computed in f64 and rounded once (iq2.py:387, :470)
         QpSteps qp4{};

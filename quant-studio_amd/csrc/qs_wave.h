@@ -95,7 +95,8 @@ struct SbPos {
     int64_t col;     // column of the lane's group start within its row
 };
 
-template <int LPS, int GROUP, int WPG = 1>
+// With LPG > 1, LPG consecutive lanes share one group of GROUP values.
+template <int LPS, int GROUP, int WPG = 1, int LPG = 1>
 QS_DEV SbPos sb_pos(int64_t n_sb, int64_t sb_per_row, int64_t stride) {
     constexpr int SPW = 64 / LPS;
     SbPos p;
@@ -106,7 +107,7 @@ QS_DEV SbPos sb_pos(int64_t n_sb, int64_t sb_per_row, int64_t stride) {
     p.valid = sb < n_sb;
     p.sb = p.valid ? sb : n_sb - 1;
     const int64_t row = p.sb / sb_per_row;
-    p.col = (p.sb % sb_per_row) * QK_K + (int64_t)p.g * GROUP;
+    p.col = (p.sb % sb_per_row) * QK_K + (int64_t)(p.g / LPG) * GROUP;
     p.elem = row * stride + p.col;
     return p;
 }

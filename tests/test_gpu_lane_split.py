@@ -17,7 +17,7 @@ COUNTS = [1, 3, 255, 2048, 2049, 4096, 4097, 6144, 6145, 12288]
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("imat", [False, True])
-@pytest.mark.parametrize("qtype", ["q2_k", "q4_k", "q5_k"])
+@pytest.mark.parametrize("qtype", ["q2_k", "q3_k", "q4_k", "q5_k", "iq4_xs"])
 def test_variants_agree_over_the_dispatch(qs, dev, qtype, imat, dtype):  # noqa: F811
     gen = torch.Generator(device="cuda").manual_seed(17)
     rows = 12300
