@@ -467,16 +467,16 @@ QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[CH / 2], 
 // smallest scores of a list and decides where they differ by
 // 64 u (sc^2 W + s2) = 2^-18 (sc^2 W + s2); the other lists (ties, and those with NaN,
 // infinite, overflowing or vanishing sums) go through the exact search, as a
-// wave-wide pass when any lane has one. A wave whose searched subgroups hold a
-// zero weight (an imatrix column that never fired) takes the exact search
-// instead of the screen: its lists tie by construction, and both passes took
-// up to 1.5 times the exact one (IQ3_XXS with a quarter of the columns zero).
-// Measured with random / a quarter zero columns, 2560x2560, before the screen and
-// code check -> now: IQ2_XXS 525 / 517 -> 453 / 513 us, IQ2_XS 423 / 417 -> 340 / 395,
-// IQ2_S 355 / 356 -> 334 / 384 (its zero columns lose 8% to the spills of the second
-// search), IQ3_XXS 465 / 461 -> 414 / 435, IQ3_S 318 / 312 -> 299 / 299. (Expanding the square to g (A g - B),
-// also three instructions, needs a bound ~100 times larger, and waves ran the
-// exact search too often: IQ2_XXS 1,633 us.) A pad entry scores like a point at
+// wave-wide pass when any lane has one. Subgroups whose entries tie whatever the
+// scale (iq_tied) take the exact search instead of the screen: screen and exact
+// search took up to 1.3 times the exact one alone.
+// Measured, bf16 1024x2560, before the screen -> now: IQ2_XXS 272 -> 233 us, IQ2_XS
+// 209 -> 169, IQ2_S 179 -> 165, IQ3_XXS 209 -> 182, IQ3_S 141 -> 124; with a constant
+// imatrix (ties; screen and exact search in brackets) IQ2_XXS 268 -> 264 (270),
+// IQ2_XS 208 -> 197 (223), IQ2_S 177 -> 188 (217), IQ3_XXS 210 -> 190 (241), IQ3_S
+// 140 -> 130 (151). (Expanding the square to g (A g - B), also three
+// instructions, needs a bound ~100 times larger, and waves ran the exact search
+// too often: IQ2_XXS 1,633 us.) A pad entry scores like a point at
 // levels 255: it can only make a list undecided (as the smallest score its
 // index is not taken).
 // The scores are non-negative, so their bits order them.
@@ -489,19 +489,15 @@ QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[CH / 2], 
 // 1,126 -> 1,088 us on normal weights, IQ2_XS 1,064 -> 1,029; IQ2_S spills 20 more
 // registers and loses a fifth, so it deals every chunk.
 //   sec: LDS, 64 words (the second smallest score of each lane's list)
+//   tied: the wave's exact search at once (uniform over the wave)
 template <int BITS, int OFF, int MAXCH, int GS, bool OWN, bool WL = false, int N>
 QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, unsigned long long* res, uint32_t* sec,
-                     const float (&xv)[N], const float (&wv)[N], float sc, uint32_t ci, bool want, bool& on) {
+                     const float (&xv)[N], const float (&wv)[N], float sc, uint32_t ci, bool want, bool& on, bool tied) {
     constexpr int NV = BITS == 2 ? 8 : 4, CH = BITS == 2 ? IQ2_CH : IQ3_CH;
     const int lane = WL ? lane_id() : (int)threadIdx.x;
     on = (ci & CI_ON_GRID) != 0;
     const bool listed = want && !on;
-    // a zero weight makes entries tie that differ in its value only, so the
-    // exact search would follow for most of such lists: it runs at once
-    float wmin = wv[OFF];
-#pragma unroll
-    for (int e = 1; e < NV; e++) wmin = fminf(wmin, wv[OFF + e]);
-    if (wave_any(listed && !(wmin > 0.0f)))
+    if (tied)
         return iq_search<BITS, NV, OFF, CH, MAXCH, WL>(T, glds, cmap, res, xv, wv, sc, ci, want, on);
     const int n = listed ? (int)(ci & 0xfffu) : 0;
     // OWN: a list's first chunk is its own lane's, loaded before the scan and
@@ -577,6 +573,31 @@ QS_DEV int iq_screen(const IqTabDev& T, const uint32_t* glds, uint8_t* cmap, uns
         gi = redo ? r : gi;
     }
     return on || want ? gi : 0;
+}
+
+// Bit s: subgroup s of some active lane has entries that tie whatever the scale, so
+// the screen would leave lists of the wave to the exact search in most steps: a
+// zero weight (an imatrix column that never fired; entries that differ in its
+// value only tie), or two values with the same magnitude and weight (entries
+// with their levels exchanged tie: 16-bit rows without an imatrix or with a
+// constant one; 1 in 100 of the bf16 subgroups of 4 and 1 in 22 of those of 8 hold
+// such a pair, so half of the waves of IQ3 and nearly all of IQ2's). Neither
+// changes over the sweep, so it is formed once.
+template <int NV, int NSUB, int N>
+QS_DEV uint32_t iq_tied(const float (&xv)[N], const float (&wv)[N], bool active) {
+    uint32_t tied = 0;
+    static_for<0, NSUB>([&](auto S) {
+        constexpr int O = NV * S;
+        float m = wv[O];
+#pragma unroll
+        for (int i = 1; i < NV; i++) {
+            m = fminf(m, wv[O + i]);
+#pragma unroll
+            for (int j = 0; j < i; j++) m = fminf(m, fabsf(xv[O + i] - xv[O + j]) + fabsf(wv[O + i] - wv[O + j]));
+        }
+        tied |= wave_any(active && !(m > 0.0f)) ? 1u << S : 0u;
+    });
+    return tied;
 }
 
 // Every subgroup whose search found no finite distance (rare: an infinite
@@ -783,6 +804,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     float scale = scale0, best = 0.0f;
     const int zero_gi = T.code0;
     int L[4] = {zero_gi, zero_gi, zero_gi, zero_gi};
+    const uint32_t tied = iq_tied<8, 4>(xval, waux, active);
 #pragma unroll 1
     for (int st = 0; st < sweep.n; st++) {
         const float inv = rdiv(sweep.v[st], eff_safe);
@@ -792,7 +814,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         uint32_t ci[4];
         iq_codes<2, 8, 4, 2>(T, xval, inv, ci, sc);
         static_for<0, 4>([&](auto S) {
-            gi[S] = iq_screen<2, 8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on);
+            gi[S] = iq_screen<2, 8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on, tied >> S & 1u);
         });
         iq_rescan<8, IQ2_CH, true>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
@@ -813,7 +835,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         uint32_t ci[4];
         iq_codes<2, 8, 4, 2>(T, xval, inv, ci, scale);
         static_for<0, 4>([&](auto S) {
-            gp[S] = iq_screen<2, 8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S], proj, on);
+            gp[S] = iq_screen<2, 8 * S, IQ2_256_MAXCH, 256, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S], proj, on, tied >> S & 1u);
         });
         iq_rescan<8, IQ2_CH, true>(T, glds, xval, waux, scale, gp);
         float sumqx, sumq2;
@@ -909,6 +931,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
     float scale = active ? gmax / 5.0f : 0.0f, best = 0.0f;
     int win[2] = {code0, code0};
     bool og[2] = {true, true};
+    const uint32_t tied = iq_tied<8, 2>(xval, waux, active);
 #pragma unroll 1
     for (int st = 0; st < sweep.n; st++) {
         const float inv = rdiv(sweep.v[st], gsafe), sc = 1.0f / inv;
@@ -916,8 +939,8 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         bool on[2];
         uint32_t ci[2];
         iq_codes<2, 8, 2, IS_S ? 0 : 1>(T, xval, inv, ci, sc);
-        gi[0] = iq_screen<2, 0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[0], true, on[0]);
-        gi[1] = iq_screen<2, 8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[1], true, on[1]);
+        gi[0] = iq_screen<2, 0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[0], true, on[0], tied & 1u);
+        gi[1] = iq_screen<2, 8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[1], true, on[1], tied & 2u);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
         iq_tree_sums<2, 8, 2>(glds, gi, w, xval, sumqx, sumq2);
@@ -941,9 +964,9 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         iq_codes<2, 8, 2, IS_S ? 0 : 1>(T, xval, inv, ci, scale);
         int r[2];
         r[0] = iq_screen<2, 0, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[0],
-                                                     need && !og[0], on);
+                                                     need && !og[0], on, tied & 1u);
         r[1] = iq_screen<2, 8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, scale, ci[1],
-                                                     need && !og[1], on);
+                                                     need && !og[1], on, tied & 2u);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, scale, r);
         if (need && !og[0]) win[0] = r[0];
         if (need && !og[1]) win[1] = r[1];
@@ -1078,6 +1101,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
         sumq2 = h2;
     };
     wave_sync();   // glds ready
+    const uint32_t tied = iq_tied<4, NSL>(xval, waux, active);
 #pragma unroll 1
     for (int st = 0; st < steps.n; st++) {
         const float inv = rdiv(steps.v[st], gsafe), sc = 1.0f / inv;
@@ -1086,7 +1110,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
         uint32_t ci[NSL];
         iq_codes<3, 4, NSL, 1>(T, xval, inv, ci, sc);
         static_for<0, NSL>([&](auto S) {
-            gi[S] = iq_screen<3, 4 * S, MAXCH, GS, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on[S]);
+            gi[S] = iq_screen<3, 4 * S, MAXCH, GS, true>(T, glds, cmap, res, sec, xval, waux, sc, ci[S], true, on[S], tied >> S & 1u);
         });
         iq_rescan<4, IQ3_CH, true>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
@@ -1116,7 +1140,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
         iq_codes<3, 4, NSL, 1>(T, xval, inv2, ci, scale);
         static_for<0, NSL>([&](auto S) {
             w2[S] = iq_screen<3, 4 * S, MAXCH, GS, true>(T, glds, cmap, res, sec, xval, waux, scale, ci[S],
-                                                          redo && (IS_S || !og[S]), on[S]);
+                                                          redo && (IS_S || !og[S]), on[S], tied >> S & 1u);
         });
         iq_rescan<4, IQ3_CH, true>(T, glds, xval, waux, scale, w2);
 #pragma unroll
