@@ -471,9 +471,9 @@ QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[CH / 2], 
 // scale (iq_tied) take the exact search instead of the screen: screen and exact
 // search took up to 1.3 times the exact one alone.
 // Measured, bf16 1024x2560, before the screen -> now: IQ2_XXS 272 -> 233 us, IQ2_XS
-// 209 -> 169, IQ2_S 179 -> 165, IQ3_XXS 209 -> 182, IQ3_S 141 -> 124; with a constant
+// 209 -> 169, IQ2_S 180 -> 148, IQ3_XXS 209 -> 182, IQ3_S 141 -> 124; with a constant
 // imatrix (ties; screen and exact search in brackets) IQ2_XXS 268 -> 264 (270),
-// IQ2_XS 208 -> 197 (223), IQ2_S 177 -> 188 (217), IQ3_XXS 210 -> 190 (241), IQ3_S
+// IQ2_XS 208 -> 197 (223), IQ2_S 177 -> 174 (217), IQ3_XXS 210 -> 190 (241), IQ3_S
 // 140 -> 130 (151). (Expanding the square to g (A g - B), also three
 // instructions, needs a bound ~100 times larger, and waves ran the exact search
 // too often: IQ2_XXS 1,633 us.) A pad entry scores like a point at
@@ -672,8 +672,10 @@ QS_DEV int sign_bits8(const float (&x)[N], float (&xval)[N]) {
 // reduced as tree_sum over the whole group: NV is a power
 // of two, so the group's pairwise tree is each subgroup's own tree followed by
 // a tree over the NSUB subgroup sums; reducing per subgroup keeps 2*NSUB
-// partials live instead of 2*N products
-template <int BITS, int NV, int NSUB, int N>
+// partials live instead of 2*N products. KEEP: w * xval stays in the sweep
+// instead of N hoisted products (IQ2_S reloaded 9 of those and 14 other spilled
+// registers in every step, one scratch latency after the other)
+template <int BITS, int NV, int NSUB, bool KEEP = false, int N>
 QS_DEV void iq_tree_sums(const uint32_t* glds, const int (&gi)[NSUB], const float (&w)[N], const float (&xval)[N],
                          float& sumqx, float& sumq2) {
     static_assert(NV * NSUB == N && (NV & (NV - 1)) == 0, "subgroups must tile the group");
@@ -685,8 +687,10 @@ QS_DEV void iq_tree_sums(const uint32_t* glds, const int (&gi)[NSUB], const floa
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             const float q = level<NV>(gl, j);
-            a[j] = (w[NV * s + j] * xval[NV * s + j]) * q;
-            b[j] = (w[NV * s + j] * q) * q;
+            float wj = w[NV * s + j];
+            if constexpr (KEEP) keep_in_register(wj);
+            a[j] = (wj * xval[NV * s + j]) * q;
+            b[j] = (wj * q) * q;
         }
         sa[s] = tree_sum(a);
         sb[s] = tree_sum(b);
@@ -890,8 +894,13 @@ template <int SRC, bool IS_S, int SQ, int WPG>
 // syncs only with itself once the grid is staged. IQ2_S (8 KB of grid, 12.4
 // KB of LDS per one-wave workgroup, 156 VGPRs: 3 waves per SIMD) runs 4
 // waves per workgroup at 6.3 KB of LDS and 128 VGPRs per wave (4 waves per
-// SIMD, 20 spilled): 6% faster. IQ2_XS fits 4 waves per SIMD in one-wave
-// workgroups already (127 VGPRs, 10.1 KB) and stays there (1% slower with 4)
+// SIMD): 6% faster. IQ2_XS fits 4 waves per SIMD in one-wave workgroups already
+// (128 VGPRs, 10.1 KB) and stays there (1% slower with 4).
+// What IQ2_S spills (16 registers) is read outside the sweep only: the
+// magnitudes kept as they are, scalar LDS bases and KEEP in the sums took the
+// sweep's reloads from 23 a step to none. bf16 16x2560 / 2560x2560: 127 / 321 ->
+// 102 / 281 us; a quarter of the imatrix columns zero 151 / 365 -> 131 / 333.
+// (KEEP in IQ2_XS, which reloads nothing: 1% slower.)
 __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S && WPG == 1 ? 3 : 4))) void k_iq2_xs_s(KArgs a, IqTabDev T, IqSteps sweep) {
     constexpr int LPS = 16, SPW = 4, BYTES = IS_S ? 82 : 74, GS = IS_S ? 1024 : 512;
     constexpr int MAXCH = IS_S ? IQ2_1024_MAXCH : IQ2_512_MAXCH;
@@ -900,7 +909,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
     __shared__ int wlds_w[WPG][SPW][16][2];
     __shared__ uint8_t cmap_w[WPG][64 * MAXCH];
     __shared__ unsigned long long res_w[WPG][64];
-    const int wave = (int)(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));     // scalar LDS bases
     IqLds<SPW, BYTES>& s = s_w[wave];
     int (*wlds)[16][2] = wlds_w[wave];
     uint8_t* cmap = cmap_w[wave];
@@ -922,6 +931,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         signs[0] = parity_fold8<0>(x, w, xval);
         signs[1] = parity_fold8<8>(x, w, xval);
     }
+    keep_in_registers(xval);
     float gmax = xval[0];
 #pragma unroll
     for (int i = 1; i < 16; i++) gmax = fmaxf(gmax, xval[i]);
@@ -943,7 +953,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
         gi[1] = iq_screen<2, 8, MAXCH, GS, !IS_S, WL>(T, glds, cmap, res, sec, xval, waux, sc, ci[1], true, on[1], tied & 2u);
         iq_rescan<8, IQ2_CH, IS_S>(T, glds, xval, waux, sc, gi);
         float sumqx, sumq2;
-        iq_tree_sums<2, 8, 2>(glds, gi, w, xval, sumqx, sumq2);
+        iq_tree_sums<2, 8, 2, IS_S>(glds, gi, w, xval, sumqx, sumq2);
         if (active && sumq2 > 0 && sumqx * sumqx > best * sumq2) {
             const float ns = sumqx / fmaxf(sumq2, F32_TINY);
             scale = ns;
@@ -973,7 +983,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
     }
     if (need) {
         float sumqx, sumq2;
-        iq_tree_sums<2, 8, 2>(glds, win, w, xval, sumqx, sumq2);
+        iq_tree_sums<2, 8, 2, IS_S>(glds, win, w, xval, sumqx, sumq2);
         if (sumq2 > 0) scale = sumqx / fmaxf(sumq2, F32_TINY);
     }
     if (active && scale < 0) {
