@@ -192,22 +192,35 @@ QS_DEV float level(const Levels<NV>& L, int e) {
 // PRUNE 0 reads the full lists.
 //
 // The check reads the position of the value between the levels instead of
-// forming the three |d|: u = max(t, 0) - level, t = 0.5*(inv*x - 1), is
-// half of x/sc minus the code's odd level, within 2^-18 while it is below 2^10
-// (inv * sc is 1 within an ulp). |u| < 1/2 - 2^-10 puts the code level's |d| at
-// most (1 - 2^-9 + 2^-17) sc, a neighbour's at least (1 + 2^-9 - 2^-17) sc, and
-// the f32 rounding of a d is below 2^-20 sc, so the strict order holds;
-// max(t, 0) drops the lower neighbour of level 0, which does not exist. Past
-// the top level, 1/2 + 2^-10 < u < 2^10 puts the next level's |d| strictly
-// below. In between, and for scales outside 2^+-100, the full list is read. A
-// NaN value counts as u = 0: every distance is then NaN, and the first entry
-// wins in either list. 9 instructions a value, 4 at half rate, for 28 that
-// compared the |d| and packed the code with integer shifts (the code is
-// summed in f32, exact below 2^24).
+// forming the three |d|: u = max(t, 0) - level, t = 0.5*(inv*x - 1), is half of
+// x/sc minus the code's odd level. Three roundings (inv * sc is 1 within an ulp,
+// the product, the sum) leave t within 2^-22 of |x/sc|. |u| < 1/2 - 2^-10 means
+// |x/sc| <= 17 (levels to 15, u below a half), so an error below 2^-17: the code
+// level's |d| is at most (1 - 2^-9 + 2^-16) sc, a neighbour's at least
+// (1 + 2^-9 - 2^-16) sc, and the f32 rounding of a d is below 2^-19 sc, so the
+// strict order holds. max(t, 0) drops the lower neighbour of level 0, which does
+// not exist. A code whose top level is the grid's (IQ3: 7) has no upper neighbour
+// there either: t ends at LMAX, and past it every lower level's exact |d| is
+// larger, so its rounded one is no smaller.
+// Past IQ2's top level (2), 1/2 + 2^-10 < u < 2^10 puts the grid's level 3
+// strictly below: near u = 1/2 |x/sc| is 6 and the bound above holds; for larger
+// u the two |d| differ by 2 sc or by 4 (u - 1/2) sc, whichever is less, where the
+// error of u (2^-22 |x/sc| = 2^-22 (5 + 2 u)) and the roundings of the two d
+// (2^-24 times |d| and 7 sc) stay below 2^-9 sc up to u = 2^10.
+// In between, and for scales outside 2^+-100, the full list is read. A NaN value
+// counts as u = 0, as does an infinite one at the end of the levels: every
+// distance is then NaN or infinite, and the first entry wins in either list
+// (the first NaN is the first entry, all being NaN, if there is one). 9 instructions a value (IQ3: 8), 4 at half rate, for 28 that compared the
+// |d| and packed the code with integer shifts (the code is summed in f32, exact
+// below 2^24).
+// IQ3's sweep puts the group's largest value past the top level in a third of
+// its steps: IQ3_XXS 182 -> 180 us and IQ3_S 124 -> 122 (1024x2560) with the
+// reduced list there, and with the magnitudes kept in registers (k_iq3).
 template <int BITS, int NV, int NSUB, int PRUNE = 0, int N>
 QS_DEV void iq_codes(const IqTabDev& T, const float (&xv)[N], float inv, uint32_t (&ci)[NSUB], float sc) {
     // all subgroups' codes first, so their cinfo loads are in flight together
-    constexpr float LMAX = BITS == 2 ? 2.0f : 7.0f;
+    constexpr float LMAX = BITS == 2 ? 2.0f : 7.0f;     // the code's largest level
+    constexpr float GMAX = BITS == 2 ? 3.0f : 7.0f;     // the grid's
     constexpr float EPS = 0x1p-10f;
     const bool prune = PRUNE > 0 && sc >= 0x1p-100f && sc <= 0x1p100f;
     int code[NSUB];
@@ -217,8 +230,9 @@ QS_DEV void iq_codes(const IqTabDev& T, const float (&xv)[N], float inv, uint32_
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             // 0.5 * fl(p - 1) = fl(0.5 p - 0.5)
-            const float t = fmaxf(__builtin_fmaf(inv * xv[NV * s + j], 0.5f, -0.5f), 0.0f);
-            const float lf = fminf(rintf(t), LMAX);
+            const float p = __builtin_fmaf(inv * xv[NV * s + j], 0.5f, -0.5f);
+            const float t = LMAX < GMAX ? fmaxf(p, 0.0f) : __builtin_amdgcn_fmed3f(p, 0.0f, LMAX);
+            const float lf = LMAX < GMAX ? fminf(rintf(t), LMAX) : rintf(t);
             sum = __builtin_fmaf(lf, (float)(1 << (BITS * j)), sum);
             if constexpr (PRUNE > 0) {
                 const float h = fabsf(t - lf) - 0.5f;
@@ -1084,6 +1098,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
     } else {
         static_for<0, NCH>([&](auto S) { signs[S] = parity_fold8<8 * S>(x, w, xval); });
     }
+    keep_in_registers(xval);               // else the sweep of IQ3_S reloads 8 spilled registers a step, 2 with it
     float gmax = xval[0];
 #pragma unroll
     for (int i = 1; i < VPL; i++) gmax = fmaxf(gmax, xval[i]);
