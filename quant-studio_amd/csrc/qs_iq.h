@@ -1059,6 +1059,16 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(IS_S &
 // ------------------------------------------------------------------
 
 
+// Superblocks up to which a launch takes the exact search alone: two waves of two
+// superblocks per SIMD (256 CUs x 4). IQ3's lists are a chunk or two, so a launch
+// this short takes as long as one wave, and the screen's merge and decision cost
+// the wave more than its cheaper chunks save; with more waves the chunks' issue is
+// the time. Measured, bf16 with imatrix, k = 256, us by screen / exactly:
+//   IQ3_XXS  16 superblocks 105 / 98  1,024 110 / 103  2,048 113 / 101
+//            4,096 120 / 116  6,144 136 / 138  8,192 157 / 165
+//   IQ3_S    16 69 / 66  1,024 74 / 70  2,048 75 / 69  4,096 81 / 80  6,144 92 / 95
+// IQ2's lists are longer: IQ2_XS 16x2560 113 us by screen, 142 exactly.
+constexpr int64_t IQ3_EXACT = 4096;
 
 // IQ3_XXS / IQ3_S (iq3_common.py:209-256, iq3_xxs.py:31-134, iq3_s.py:31-140)
 // with LPG lanes per 32-value group: each lane holds 32/LPG values (its
@@ -1126,7 +1136,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LPG == 4 ? 6
         sumq2 = h2;
     };
     wave_sync();   // glds ready
-    const uint32_t tied = iq_tied<4, NSL>(xval, waux, active);
+    const uint32_t tied = a.n_units <= IQ3_EXACT ? ~0u : iq_tied<4, NSL>(xval, waux, active);
 #pragma unroll 1
     for (int st = 0; st < steps.n; st++) {
         const float inv = rdiv(steps.v[st], gsafe), sc = 1.0f / inv;

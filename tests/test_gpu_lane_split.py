@@ -42,3 +42,20 @@ def test_variants_agree_over_the_dispatch(qs, dev, qtype, imat, dtype):  # noqa:
     for n in COUNTS:
         assert torch.equal(fn(x[:n]).cpu(), whole[:n]), n
         assert torch.equal(fn(x[rows - n:]).cpu(), whole[rows - n:]), n
+
+
+@pytest.mark.parametrize("imat", [False, True])
+@pytest.mark.parametrize("qtype", ["iq3_xxs", "iq3_s"])
+def test_iq3_agrees_over_its_line(qs, dev, qtype, imat):  # noqa: F811
+    """Few superblocks take the exact search alone: both sides of the line."""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x = (torch.randn(4200, 256, generator=gen, device=dev) * 0.02).to(torch.bfloat16)
+    x[3] = 0
+    x[4, 64:96] = x[4, 64]
+    qw = torch.exp(torch.randn(256, generator=gen, device=dev)) if imat else None
+    fn = qs.QUANT_TYPES[qtype].make_kernel(dev, qw)
+    whole = fn(x).cpu()
+    ref = oracle.quantize(qtype, x[:400].float().cpu().numpy(), None if qw is None else qw.cpu().numpy())
+    assert np.array_equal(whole[:400].numpy(), ref)
+    for n in (1, 3, 4095, 4096, 4097):
+        assert torch.equal(fn(x[:n]).cpu(), whole[:n]), n
