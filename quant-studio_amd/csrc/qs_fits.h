@@ -134,9 +134,12 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
             this_min = 0.0f;
         }
         float den_acc = mx - this_min;
-        // only a candidate that can be accepted has to be exact
+        // only a candidate that can be accepted has to be exact. q_hi keeps a NaN
+        // (v_maximum3_f32; a quotient of an overflowed numerator, where `/` gives an
+        // infinity), which then fails the test; fminf drops it
         const bool live = D > 0;
-        const float q_lo = fminf(fminf(q_s, q_m), den_acc), q_hi = fmaxf(fmaxf(q_s, q_m), den_acc);
+        const float q_lo = fminf(fminf(q_s, q_m), den_acc);
+        const float q_hi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(q_s, q_m), den_acc);
         const bool out = live && !(q_lo >= LO && q_hi <= HI && D >= DLO && D <= DHI);
         if (wave_any(out)) {
             this_scale = num_s / Dsafe;

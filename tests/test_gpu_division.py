@@ -59,3 +59,44 @@ def test_scales_across_the_division_range(qs, dev, qtype, imat):  # noqa: F811
     fn = qs.QUANT_TYPES[qtype].make_kernel(dev, None if qw is None else torch.from_numpy(qw))
     got = fn(torch.from_numpy(xb).to(dev)).cpu().numpy()
     assert np.array_equal(got, oracle.quantize(qtype, xb, qw))
+
+
+def four_squares(n: int) -> list[int]:
+    for a in range(int(n**0.5), 0, -1):
+        for b in range(int((n - a * a) ** 0.5), -1, -1):
+            r = n - a * a - b * b
+            for c in range(int(r**0.5), -1, -1):
+                d = int((r - c * c) ** 0.5)
+                if a * a + b * b + c * c + d * d == n:
+                    return [a, b, c, d]
+    raise ValueError(n)
+
+
+@pytest.mark.parametrize("n", [1, 2100, 4200])
+def test_minimum_that_overflows(qs, dev, n):  # noqa: F811
+    """A candidate whose minimum is +inf (sum_l2 sum_x overflows: weights of
+    both signs that cancel in sum_w and sum_l, so D and the scale stay small) is
+    fitted again with a minimum of 0 (kq_common.py:77-80) and can be accepted."""
+    groups = [
+        ([2.0, 0.5625, 1.46875, 1.140625, 1.796875, 0.890625, 0.8125, 0.609375, 0.46875, 1.296875], [1, -2, -2, 2, -2]),
+        ([2.0, 0.09375, 0.53125, 0.125, 0.078125, 1.109375, 0.375, 0.15625, 1.828125, 0.296875], [2, -4, -2, 1, -2]),
+        ([2.0, 0.125, 1.203125, 0.296875, 0.109375, 1.65625, 0.796875, 1.734375, 1.484375, 0.40625], [-1, -2, -1, -1, 4]),
+    ]
+    rng = np.random.default_rng(2)
+    for values, signs in groups:
+        # multiples of 2^7 elsewhere whose squares sum to 2^36: every root is 2^14 and
+        # the group's weights are exact (and no other group of the wave is out of range)
+        m = np.rint(rng.standard_normal(240) * 110).astype(np.int64)
+        rest = 2**22 - int((m[:236] ** 2).sum())
+        m[236:] = four_squares(rest)
+        x = np.zeros((1, 256), np.float32)
+        x[0, 16:] = m * 128
+        x[0, :10] = values
+        qw = np.full(256, 2.0**-14, np.float32)
+        qw[:16] = 0
+        qw[0:10:2] = np.asarray(signs) * 2.0**52
+        qw[1:11:2] = -np.asarray(signs) * 2.0**52
+        qw[10] = 2.0**-54
+        fn = qs.QUANT_TYPES["q2_k"].make_kernel(dev, torch.from_numpy(qw))
+        got = fn(torch.from_numpy(x).to(dev).repeat(n, 1)).cpu().numpy()
+        assert (got == oracle.quantize("q2_k", x, qw)).all()
