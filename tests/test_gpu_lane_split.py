@@ -75,6 +75,9 @@ def edge_runs(imat: bool):
     big[4:6, 600] = 2.0e36
     big[6:8, 1004] = 3.3e38
     yield "values near FLT_MAX", big, q
+    sparse = x * (rng.random(x.shape) < 0.1)
+    sparse[4:, ::512] = x[4:, ::512]
+    yield "mostly zero values", np.concatenate([sparse, x[:3]]).astype(np.float32), q
     scale = np.repeat([1e-13, 3e-15, 1.2e-15, 8e-16], 2)[:, None]
     yield "tiny values", (rng.standard_normal((8, k)) * scale).astype(np.float32), q
     if not imat:
