@@ -85,8 +85,11 @@ QS_DEV QkxResult qkx_fit(const float (&x)[N], const float (&w)[N], const Steps& 
     // are then at least 2^-96 and at most 2^120, the inverse scales (the candidates'
     // numerators are 0.5 .. 33) within 2^+-61. D is about the square of a group's
     // weights, so DHI takes imatrix entries of up to about 2^27 (with 2^36, entries
-    // beyond 2^15 divided plainly: Q2_K 1024x2560 66 us instead of 60).
-    constexpr float LO = 0x1p-36f, HI = 0x1p60f, DLO = 0x1p-60f, DHI = 0x1p60f;
+    // beyond 2^15 divided plainly: Q2_K 1024x2560 66 us instead of 60). Where DHI is
+    // HI the compiler tests both with one compare: 3% faster with 8 values a lane
+    // (Q4_K imatrix 400x2560 32.6 -> 31.5 us), but 1.5% slower with 4 (16x512 20.4 ->
+    // 20.8), which keep two.
+    constexpr float LO = 0x1p-36f, HI = 0x1p60f, DLO = 0x1p-60f, DHI = N == 4 ? 0x1p59f : HI;
     float y = recip(den);                     // of the current range
     // lanes whose current range needs `/` (a mask, so it stays in scalar registers)
     uint64_t far = wave_mask(!(den >= LO && den <= HI));
