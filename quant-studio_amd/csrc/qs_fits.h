@@ -650,10 +650,10 @@ QS_DEV void iq4_pack(const float (&x)[32], float id, const Iq4Tab& t, uint32_t (
 
 // _search_scales_eager iq4_xs.py:52-76 for one block of 32. The two sums of
 // a candidate run left to right (seq_sum's order) over terms staged CH values
-// at a time: CH = 16 holds 121-126 VGPRs instead of 140-168, which with the
-// imatrix weights taken 8 at a time gives the imatrix kernels a fourth wave
-// per SIMD (6-7% faster); the kernels without imatrix were 4% slower at 4
-// waves and stage all 32 (CH = 32, 3 waves).
+// at a time: the imatrix kernels hold 128 VGPRs with CH = 16, a fourth wave per
+// SIMD (6-7% faster; IQ4_XS at one lane per block spills 8, 14 with the AMD host's
+// maps). The kernels without imatrix hold 81-106 with all 32 staged (CH = 32), four
+// waves as well.
 // LPG > 1: the LPG lanes c = 0 .. LPG - 1 of a block all hold it, lane c forms the
 // sums of trials c, c + LPG, ... (a trial does not depend on earlier accepts),
 // they meet in xch (32 floats of LDS), and every lane runs the accept chain in

@@ -296,8 +296,10 @@ __device__ __attribute__((noinline)) int iq_argmin_scan_call(const uint16_t* nbr
 
 // First minimum of one chunk (CH list slots from slot CH*kc) as a 64-bit key
 // (distance bits, list position, grid index); slots past the list end (o_n)
-// are masked out. Every slot is evaluated (padding holds index 0, a valid
-// grid point), without branches. IQ2: slots are visited in list order, so a
+// are masked out. Every slot is evaluated, without branches: padding holds index
+// GS, the pad point that stage_levels adds to the GS grid points in LDS (so glds
+// holds GS + 1 points, and a reader masks by the list's length or rejects GS; it
+// is no index of T.grid). IQ2: slots are visited in list order, so a
 // strict `d2 < best` keeps the first minimum and the key is built once per
 // chunk (4-7% faster); a chunk with no finite distance returns ~0 (as if it
 // held no candidate: with no finite distance anywhere in the list the search
