@@ -497,13 +497,12 @@ QS_DEV void iq_chunk_screen(const uint32_t* glds, const uint32_t (&wd)[CH / 2], 
 // index is not taken).
 // The scores are non-negative, so their bits order them.
 // The chunk arithmetic was about 70% of the searches' instructions. Measured with
-// imatrix: IQ2_XXS bf16 2560x9728 1,177 -> 1,023 us (722 M VALU instructions a
-// launch instead of ~940 M; its 3 waves per SIMD now wait on memory and LDS a
-// third of their cycles), IQ2_S 9728x2560 1,082 -> 1,036, IQ2_XS, with the shorter
-// code check, 1,312 -> 1,030; IQ3_XXS 9728x2560 1,449 -> 1,317, 1024x2560 192 -> 177,
-// IQ3_S 9728x2560 962 -> 947. With OWN against dealing every chunk: IQ2_XXS
-// 1,126 -> 1,088 us on normal weights, IQ2_XS 1,064 -> 1,029; IQ2_S spills 20 more
-// registers and loses a fifth, so it deals every chunk.
+// imatrix, bf16 9728x2560, exact search alone -> now (with the code check by position):
+// IQ2_XXS 1,255 -> 1,085 us (its 3 waves per SIMD wait on memory and LDS a third of
+// their cycles), IQ2_XS 1,277 -> 1,039, IQ2_S 1,056 -> 892, IQ3_XXS 1,576 -> 1,402,
+// IQ3_S 1,090 -> 942. With OWN against dealing every chunk: IQ2_XXS 1,126 -> 1,088 us
+// on normal weights, IQ2_XS 1,064 -> 1,029; IQ2_S, measured before its sweep was free
+// of reloads, lost a fifth to 20 more spilled registers and deals every chunk.
 //   sec: LDS, 64 words (the second smallest score of each lane's list)
 //   tied: the wave's exact search at once (uniform over the wave)
 template <int BITS, int OFF, int MAXCH, int GS, bool OWN, bool WL = false, int N>
